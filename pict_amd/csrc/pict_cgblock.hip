@@ -1,0 +1,887 @@
+// pict_cgblock.hip -- single-reduction CG with a system's whole state on chip, one large workgroup per
+// compute unit (one right-hand side, norm-2 criteria, rows of at most 7 entries).
+//
+// The recurrences of k_cg1 / k_cg_local (pict_solve.hip: Chronopoulos & Gear 1989, the iterates of
+// cgSolveGPU, cg_solver_kernel.cu:114-456).  A workgroup of 512 threads owns up to 512*RPT rows; the
+// matrix entries, w and s of a thread's rows stay in its registers, r in LDS (x and p in registers, in
+// LDS and memory for the largest instances), so an iteration reads no matrix and no vector from memory.
+//
+// Other workgroups' rows ("halo").  A product needs r' of rows that another workgroup owns.  r' follows
+// from r, s and w by two fmas, so a reader keeps its own copy of the halo rows' r (LDS) and s (registers),
+// advances them with the owner's fma sequence (bitwise the owner's values), and only w travels: one word
+// per halo row and iteration, as agent-scope atomics that need no L2 writeback or invalidation.  FP32
+// words carry their iteration, so a reader waits on the data itself while the reduction is under way; FP64
+// words cannot, so there a workgroup waits for its stores before it posts its partial sums.
+// Halo rows are found in the first pass: every foreign column marks its tile of 8 rows in a bitmap (LDS),
+// a scan numbers the marked tiles, and a row's register entry is the LDS offset of the column.
+//
+// Rows of a workgroup.  Rows in order for 5-entry (2-D) systems.  For 7-entry (3-D) systems a contiguous
+// chunk would have most of its neighbours a plane away in other workgroups (192x96x96 on 256 workgroups:
+// 14,200 halo rows for 6,912 own rows), so the grid's line length and plane are read off the matrix (the
+// column offsets -d3, -d2, -1, 0, 1, d2, d3 of an interior row) and a workgroup owns a block of whole
+// lines (6 x 6 lines: 4,608 halo rows).  The mapping is a bijection of the rows whatever the matrix is:
+// a wrong guess costs halo rows, never correctness.
+//
+// What bounds it: an iteration is one trip of the partial sums through memory (about 1.3 us between the XCDs for up to
+// 128 workgroups, 2 for 256), three workgroup barriers, and per row 0.25 us of LDS gathers and FP64 sums on a unit that
+// holds 14 of them per thread.  At 192 x 96 x 96 it takes 7.8 us where streaming the system takes 40 (184 MB at 4.6
+// TB/s); figures for other sizes stand at plan_block (pict_solve.hip).
+//
+// A system of several workgroups that this kernel cannot hold (a longer row, too many halo rows, no block
+// partition) is left alone: the kernel sets ctl->zero_all ("not solved") before it writes x, and the general
+// kernel queued behind it runs; otherwise that kernel returns at once.
+#include <hip/hip_runtime.h>
+
+#include <cmath>
+#include <type_traits>
+
+#include "pict_krylov.hpp"
+
+namespace pict {
+
+constexpr int kTile = 8;  // rows of a halo tile
+
+// base[i] through a scalar base and a 32-bit byte offset (one address register per load, not two): every array of a
+// system this kernel takes is below 4 GiB
+template <typename E>
+__device__ __forceinline__ E *elem(E *base, unsigned i) {
+    using Byte = std::conditional_t<std::is_const_v<E>, const char, char>;
+    return reinterpret_cast<E *>(reinterpret_cast<Byte *>(base) + (size_t)(i * (unsigned)sizeof(E)));
+}
+
+// Owner and local index of the rows of a system.
+struct BlockMap {
+    int n, nwg;                // workgroups that own rows
+    int brick;                 // 0: rows in order, 1: blocks of a x b lines
+    int nx, ny, nz, a, b, nby;
+    float inx, iny, ia, ib, inby;  // reciprocals
+};
+// floor(v / d) from d's rounded reciprocal, for v < 2^21 (every position of a system this kernel takes): the exact
+// (v + 1/2) / d lies at least 1 / (2 d) from an integer, the two roundings move it by less than v / d * 2^-22
+__device__ __forceinline__ unsigned block_div(unsigned v, float inv) { return (unsigned)(((float)v + 0.5f) * inv); }
+
+template <int C>
+__device__ __forceinline__ int block_row(const BlockMap &m, unsigned bid, unsigned li) {
+    if (!m.brick) {
+        const int i = (int)(bid * (unsigned)C + li);
+        return i < m.n ? i : -1;
+    }
+    const unsigned line = block_div(li, m.inx), x = li - line * (unsigned)m.nx;
+    const unsigned lz = block_div(line, m.ia), ly = line - lz * (unsigned)m.a;
+    const unsigned bz = block_div(bid, m.inby), by = bid - bz * (unsigned)m.nby;
+    const unsigned y = by * (unsigned)m.a + ly, z = bz * (unsigned)m.b + lz;
+    if (lz >= (unsigned)m.b || y >= (unsigned)m.ny || z >= (unsigned)m.nz) return -1;
+    const int i = (int)((z * (unsigned)m.ny + y) * (unsigned)m.nx + x);
+    return i < m.n ? i : -1;
+}
+// position of row c: owner * C + local index
+template <int C>
+__device__ __forceinline__ unsigned block_pos(const BlockMap &m, unsigned c) {
+    if (!m.brick) return c;
+    const unsigned line = block_div(c, m.inx), x = c - line * (unsigned)m.nx;
+    const unsigned z = block_div(line, m.iny), y = line - z * (unsigned)m.ny;
+    const unsigned by = block_div(y, m.ia), ly = y - by * (unsigned)m.a;
+    const unsigned bz = block_div(z, m.ib), lz = z - bz * (unsigned)m.b;
+    return (bz * (unsigned)m.nby + by) * (unsigned)C + (lz * (unsigned)m.a + ly) * (unsigned)m.nx + x;
+}
+
+// The row mapping, by all threads of a workgroup (every workgroup finds the same one); key: LDS scratch.
+template <int T, int C, int NZ>
+__device__ __forceinline__ void block_map(const int32_t *row, const int32_t *col, int n, int nwg, BlockMap &m,
+                                          unsigned *key) {
+    const int t = (int)threadIdx.x;
+    if (t == 0) {
+        m.n = n;
+        m.brick = 0;
+        m.nwg = (n + C - 1) / C;
+        key[0] = key[1] = 0xffffffffu;
+    }
+    __syncthreads();
+    if constexpr (NZ == 7) {
+        // lines and planes: the first of T rows spread over the system (at varying places in their lines) with the
+        // offsets of an interior row
+        const int i = (int)((((long long)n * (2 * t + 1)) / (2 * T) + 37 * t) % n);
+        int d2 = 0, d3 = 0;
+        const int rs = row[i];
+        if (row[i + 1] - rs == 7 && col[rs + 3] == i && col[rs + 4] == i + 1 && col[rs + 2] == i - 1) {
+            d2 = col[rs + 5] - i;
+            d3 = col[rs + 6] - i;
+            const bool ok = col[rs + 1] == i - d2 && col[rs] == i - d3 && d2 >= 4 && d3 > d2 && d3 % d2 == 0;
+            if (ok) atomicMin(&key[0], (unsigned)t);
+        }
+        __syncthreads();
+        const unsigned who = key[0];
+        if (who != 0xffffffffu && (unsigned)t == who) {
+            m.nx = d2;
+            m.ny = d3 / d2;
+            m.nz = (int)(((long long)n + d3 - 1) / d3);
+        }
+        __syncthreads();
+        if (who != 0xffffffffu) {
+            // blocks of a x b lines that fit a workgroup, at most nwg of them, with the fewest halo lines
+            const int nx = m.nx, ny = m.ny, nz = m.nz;
+            int a = 0, b = 0, nby = 0, nbz = 0;
+            if (t < ny && (long long)nx * (t + 1) <= C) {
+                nby = (ny + t) / (t + 1);
+                a = (ny + nby - 1) / nby;
+                b = min(C / (nx * a), nz);
+                nbz = (nz + b - 1) / b;
+                b = (nz + nbz - 1) / nbz;
+                const int halo = (nby > 1 ? b : 0) + (nbz > 1 ? a : 0);
+                if ((long long)nby * nbz <= nwg) atomicMin(&key[1], ((unsigned)halo << 16) | (unsigned)t);
+            }
+            __syncthreads();
+            if (key[1] != 0xffffffffu && (key[1] & 0xffffu) == (unsigned)t) {
+                m.a = a;
+                m.b = b;
+                m.nby = nby;
+                m.nwg = nby * nbz;
+                m.inx = 1.0f / (float)nx;
+                m.iny = 1.0f / (float)ny;
+                m.ia = 1.0f / (float)a;
+                m.ib = 1.0f / (float)b;
+                m.inby = 1.0f / (float)nby;
+                m.brick = 1;
+            }
+            __syncthreads();
+        }
+    }
+}
+
+// Wave totals of two sums at once: every lane of the lower half gets v0's, of the upper half v1's (the halves are
+// swapped so that each carries one value, then both go through the same five steps).
+__device__ __forceinline__ double wave_sum2(double v0, double v1) {
+    auto swap32 = [](double &x, double &y) {
+        const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(x), __double2loint(y), false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(x), __double2hiint(y), false, false);
+        x = __hiloint2double((int)hi[0], (int)lo[0]);
+        y = __hiloint2double((int)hi[1], (int)lo[1]);
+    };
+    swap32(v0, v1);
+    double v = v0 + v1;
+    v += dpp_d<0xB1>(v);   // quad_perm [1,0,3,2]
+    v += dpp_d<0x4E>(v);   // quad_perm [2,3,0,1]
+    v += dpp_d<0x124>(v);  // row_ror:4
+    v += dpp_d<0x128>(v);  // row_ror:8
+    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(v), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(v), false, false);
+    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+
+// Totals of one generation over the workgroups' tagged pairs (lane l: workgroups l, l + 64, ... in that
+// order, then across the lanes): the same bits in every workgroup.  At most 256 workgroups; B of a lane's in flight.
+template <int B>
+__device__ __forceinline__ bool block_poll(const u64 *part, unsigned nwg, unsigned gen, bool max1, double &t0,
+                                           double &t1) {
+    const unsigned lane = threadIdx.x & 63;
+    const u64 *set = part + (size_t)(gen & 1u) * nwg * 2;
+    double v0, v1;
+    unsigned spins = 0;
+    for (;;) {
+        bool ready = true;
+        v0 = v1 = 0.0;
+#pragma unroll
+        for (int b = 0; b < 4; b += B) {
+            if (64u * b >= nwg) continue;
+            u64 u[B][2];
+#pragma unroll
+            for (int j = 0; j < B; ++j) {
+                if (64u * (b + j) >= nwg) continue;
+                const unsigned w = lane + 64u * (b + j);
+                const u64 *p = set + (size_t)(w < nwg ? w : 0u) * 2;
+                u[j][0] = ld_coh(p);
+                u[j][1] = ld_coh(p + 1);
+            }
+#pragma unroll
+            for (int j = 0; j < B; ++j) {
+                if (lane + 64u * (b + j) >= nwg) continue;
+                ready = ready && partial_ready(u[j][0], gen) && partial_ready(u[j][1], gen);
+                v0 += partial_value(u[j][0]);
+                const double q = partial_value(u[j][1]);
+                v1 = max1 ? fmax(v1, q) : v1 + q;
+            }
+        }
+        if (__all(ready)) break;
+        if (++spins > kSpinLimit) return false;
+    }
+    if (max1) {
+        t0 = wave_reduce_dpp<false>(v0);
+        t1 = wave_reduce_dpp<true>(v1);
+    } else {
+        const double v = wave_sum2(v0, v1);
+        t0 = lane_d(v, 0);
+        t1 = lane_d(v, 32);
+    }
+    return true;
+}
+
+// The scalar step of cg_run_update (pict_krylov.hpp) for the norm-2 criteria without best-result bookkeeping; the
+// criterion's square root is taken only near the tolerance and at the end (final_res: block_run_end).
+template <typename R>
+__device__ __forceinline__ void block_run_update(const SolveArgs<R> &a, CgRun &st, double gam, double delta, int it) {
+    const double beta_n = gam * st.inv_rho;
+    const double den_n = fma(-beta_n * beta_n, st.den, delta);
+    st.used = it;
+    const double near = gam * (a.crit_scale * a.crit_scale);
+    if (!(near > 1.0001 * a.tol * a.tol) || !(near < 1e300)) {
+        const double crit = sqrt(gam) * a.crit_scale;
+        const bool finite = isfinite(crit);
+        if (!finite || crit < a.tol) {
+            st.converged = st.finite = finite;
+            st.final_res = crit;
+            st.active = 0;
+            return;
+        }
+    }
+    st.alpha = gam * rcp64(den_n);
+    st.beta = beta_n;
+    st.den = den_n;
+    st.rho = gam;
+    st.inv_rho = rcp64(gam);
+}
+template <typename R>
+__device__ __forceinline__ void block_run_end(const SolveArgs<R> &a, CgRun &st) {
+    if (st.active && st.used >= 0) st.final_res = sqrt(st.rho) * a.crit_scale;  // the iteration limit
+}
+
+// ONE: the system fits one workgroup: no exchange, no halo, and every thread runs the scalar step on the
+// wave totals (two workgroup barriers per iteration instead of three and no trip through memory).
+// HPT: halo rows per thread of waves 1..
+// BIG: more rows per thread than the registers hold vectors of: p, s and the halo's s in LDS, and x in memory (4 bytes
+// per row each way, while the workgroup waits for the totals).
+template <typename R, int T, int RPT, int NZ, int HPT, bool BIG, bool ONE>
+__device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
+    constexpr int kBW = T / 64;
+    constexpr int kBF = T - 64;  // threads that hold halo rows: waves 1.. (wave 0 polls the reduction)
+    constexpr int C = T * RPT;
+    constexpr int H = ONE ? 0 : kBF * HPT;
+    constexpr int LR = ONE ? C : C + (H > C / 2 ? H : C / 2);  // also the set-up's bitmap and tile numbers
+    constexpr int NO = NZ - 1, NI = (NO + 1) / 2;
+    constexpr bool kTagged = Pub<R>::kTagged;
+    static_assert((C + H) * sizeof(R) <= 65536, "LDS offsets are 16 bits");
+    __shared__ R lr[LR];  // r of the own rows, then of the halo rows
+    // BIG: p, s, then s and the fetched w of the halo rows, then w of WL rows per thread
+    constexpr int WL = BIG ? 4 : 0;
+    __shared__ R lps[BIG ? 2 * C + 2 * H + WL * T : 1];
+    __shared__ int ltile[ONE ? 1 : H / kTile + 1];  // halo tile: position of its first row / kTile
+    __shared__ double wsum[2][2 * kBW];  // by generation parity: the waves' first sums, then their second
+    __shared__ int scan[kBW];
+    __shared__ unsigned key[2];
+    __shared__ BlockMap m;
+    __shared__ int s_over, s_err;
+    struct Step {
+        double alpha, beta;
+        int active;
+    };
+    __shared__ Step bc;
+    // the wave number as a scalar: a wave takes its branch alone, without the other branch's waits
+    const int t = (int)threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    int herr = 0;
+    if (t == 0) s_over = s_err = 0;
+    if constexpr (ONE) {
+        if (t == 0) m = BlockMap{a.n, 1};
+        __syncthreads();
+    } else {
+        block_map<T, C, NZ>(a.row, a.col, a.n, (int)a.nwg, m, key);
+        __syncthreads();
+        if (bid >= (unsigned)m.nwg) return;
+    }
+    const unsigned nwg = (unsigned)m.nwg;
+    const unsigned first = bid * (unsigned)C;  // position of the first own row
+    using PubT = decltype(Pub<R>::base);
+    const Pub<R> pub{reinterpret_cast<PubT>(a.pub), (int)(a.nwg * (unsigned)C)};  // w by position, two parities
+    auto put_row = [&](int par, unsigned pos, R v, unsigned tag) {
+        PubT base = pub.base + (size_t)par * pub.n;
+        if constexpr (kTagged) st_coh(elem(base, pos), ((u64)tag << 32) | (u64)__float_as_uint(v));
+        else st_coh(elem(base, pos), v);
+    };
+    int *mark = reinterpret_cast<int *>(a.p0);  // tiles that another workgroup reads (stamped with a.salt)
+    int nh = 0;                                 // halo rows (a multiple of kTile)
+
+    // ---- halo tiles ----
+    if constexpr (!ONE) {
+        unsigned *bits = reinterpret_cast<unsigned *>(lr);
+        const int nw = (int)(nwg * (unsigned)(C / (kTile * 32)));
+        unsigned short *base = reinterpret_cast<unsigned short *>(bits + nw);
+        for (int k = t; k < nw; k += T) bits[k] = 0;
+        __syncthreads();
+        for (int q = 0; q < RPT; ++q) {
+            const int i = block_row<C>(m, bid, (unsigned)(t + q * T));
+            if (i < 0) continue;
+            const int rs = a.row[i], re = a.row[i + 1];
+            bool diag = false;
+            for (int e = rs; e < re; ++e) {
+                const unsigned c = (unsigned)a.col[e];
+                diag |= (int)c == i;
+                const unsigned pos = block_pos<C>(m, c);
+                if (pos - first >= (unsigned)C) atomicOr(&bits[pos / (kTile * 32)], 1u << ((pos / kTile) & 31));
+            }
+            if (re - rs > NO + (diag ? 1 : 0)) s_over = 1;
+        }
+        __syncthreads();
+        const int per = (nw + T - 1) / T, k0 = min(t * per, nw), k1 = min(k0 + per, nw);
+        int cnt = 0;
+        for (int k = k0; k < k1; ++k) cnt += __popc(bits[k]);
+        int inc = cnt;
+#pragma unroll
+        for (int off = 1; off < 64; off *= 2) {
+            const int o = __shfl_up(inc, off, 64);
+            if (lane >= off) inc += o;
+        }
+        if (lane == 63) scan[wave] = inc;
+        __syncthreads();
+        int start = inc - cnt, total = 0;
+        for (int w = 0; w < kBW; ++w) {
+            if (w < wave) start += scan[w];
+            total += scan[w];
+        }
+        if (total * kTile > H) {
+            if (t == 0) s_over = 1;
+        }
+        for (int k = k0; k < k1; ++k) {
+            base[k] = (unsigned short)start;
+            for (unsigned b = bits[k]; b; b &= b - 1) {
+                const int tile = k * 32 + __ffs((int)b) - 1;
+                if (start < H / kTile) ltile[start] = tile;
+                st_coh(mark + tile, a.salt);
+                ++start;
+            }
+        }
+        nh = min(total * kTile, H);
+        __syncthreads();
+        // a thread's unused halo slots repeat its first one
+        for (int k = t; k < H / kTile; k += T)
+            if (k * kTile >= nh) ltile[k] = (k % (kBF / kTile)) * kTile < nh ? ltile[k % (kBF / kTile)] : 0;
+        __syncthreads();
+    }
+
+    // ---- rows into registers; r0 = b - A x0 ----
+    R dv[RPT], val[RPT][NO], w[RPT], s[BIG ? 1 : RPT], x[BIG ? 1 : RPT], p[BIG ? 1 : RPT];
+    unsigned idx[RPT][NI];
+    unsigned longm = 0;  // bit q: row q is read from memory (ONE)
+    double acc0 = 0.0, acc1 = 0.0;
+#pragma unroll
+    for (int q = 0; q < RPT; ++q) {
+        const int li = t + q * T;
+        const int i = block_row<C>(m, bid, (unsigned)li);
+        const int ii = i < 0 ? 0 : i;
+        const int rs = *elem(a.row, ii);
+        int len = i < 0 ? 0 : *elem(a.row, ii + 1) - rs;
+        if constexpr (ONE) {
+            // a row of more entries than the registers hold is read from memory in every product
+            bool diag = false;
+            for (int e = 0; len >= NZ && e < NZ; ++e) diag |= a.col[rs + e] == ii;
+            if (len > NO + (diag ? 1 : 0)) {
+                longm |= 1u << q;
+                len = 0;
+            }
+        }
+        len = min(len, NZ);
+        const R x0 = i < 0 ? R(0) : *elem(a.x, ii), bv = i < 0 ? R(0) : *elem(a.b, ii);
+        // The row's entries around its diagonal: up to NO / 2 before it end at slot NO / 2 - 1, those after it start at
+        // slot NO / 2, so that a product adds them in the row's order (rows with more on one side, such as those whose
+        // neighbours wrap around, fill the slots in order).  Slots without an entry hold the own column with value 0.
+        const int last = rs + max(len, 1) - 1;
+        int pd = NZ;  // entry of the diagonal
+#pragma unroll
+        for (int e = NZ - 1; e >= 0; --e) pd = e < len && *elem(a.col, min(rs + e, last)) == ii ? e : pd;
+        const bool centred = pd <= NO / 2 && len - 1 - pd <= NO / 2;
+        auto value = [&](int k) { return *elem(a.val, a.perm ? *elem(a.perm, k) : k); };
+        dv[q] = pd < len ? value(rs + pd) : R(0);
+        R sum = 0;
+#pragma unroll
+        for (int j = 0; j < NI; ++j) idx[q][j] = 0;
+#pragma unroll
+        for (int j = 0; j < NO; ++j) {
+            const int e = centred ? j - NO / 2 + pd + (j >= NO / 2 ? 1 : 0) : j + (j >= pd ? 1 : 0);
+            const bool in = e >= 0 && e < len;
+            const int k = in ? rs + e : last;
+            const int cj = in ? *elem(a.col, k) : ii;
+            val[q][j] = in ? value(k) : R(0);
+            if (j == NO / 2) sum += dv[q] * *elem(a.x, ii);
+            sum += val[q][j] * *elem(a.x, cj);
+            const unsigned pos = block_pos<C>(m, (unsigned)cj);
+            unsigned l = pos - first;
+            if constexpr (!ONE) {
+                const unsigned *bits = reinterpret_cast<const unsigned *>(lr);
+                const unsigned short *base =
+                    reinterpret_cast<const unsigned short *>(bits + nwg * (unsigned)(C / (kTile * 32)));
+                const unsigned k = pos / (kTile * 32), bit = (pos / kTile) & 31;
+                const unsigned slot = base[k] + (unsigned)__popc(bits[k] & ((1u << bit) - 1u));
+                l = l < (unsigned)C ? l : (unsigned)C + min(slot * kTile + pos % kTile, (unsigned)(H - 1));
+            }
+            l = cj == ii ? (unsigned)li : l;  // (a row without entries has no position)
+            idx[q][j / 2] |= (l * (unsigned)sizeof(R)) << (16 * (j & 1));
+            if constexpr (BIG) asm volatile("" : "+v"(idx[q][j / 2]));  // one entry after the other (registers)
+        }
+        if constexpr (ONE)
+            if (longm >> q & 1u)
+                for (int e = rs; e < a.row[ii + 1]; ++e) sum += a.val[a.perm ? a.perm[e] : e] * a.x[a.col[e]];
+        const R rv = bv - sum;
+        w[q] = rv;  // until the bitmap in lr has been read
+        if constexpr (BIG) {
+            lps[li] = lps[C + li] = R(0);
+        } else {
+            x[q] = x0;
+            p[q] = s[q] = R(0);
+        }
+        if constexpr (!ONE) put_row(1, first + li, rv, 1u);  // every row: the marks are not known yet
+        acc0 += (double)rv * (double)rv;
+        acc1 = fmax(acc1, fabs((double)bv));
+        // a row is finished before the next one is begun (else the unrolled rows' loads and index arithmetic overlap
+        // and spill)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) asm volatile("" : "+v"(idx[q][j]));
+#pragma unroll
+        for (int j = 0; j < NO; ++j) asm volatile("" : "+v"(val[q][j]));
+        asm volatile("" : "+v"(dv[q]), "+v"(w[q])::"memory");
+        if constexpr (RPT >= 8) __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (!ONE)
+        if (s_over) acc1 = INFINITY;
+    __syncthreads();  // the bitmap has been read
+#pragma unroll
+    for (int q = 0; q < RPT; ++q) {
+        lr[t + q * T] = w[q];
+        w[q] = R(0);  // (rows in LDS: written by the first product before they are read)
+    }
+
+    // the workgroup's totals from the waves' (lane l takes entry l, then across the lanes)
+    auto wg_totals = [&](int par, bool max1, double &g0, double &g1) {
+        double v = wsum[par][lane & (2 * kBW - 1)];
+        const bool mx = max1 && (lane & kBW);
+        auto op = [&](double x, double y) { return mx ? fmax(x, y) : x + y; };
+        v = op(v, dpp_d<0xB1>(v));  // quad_perm [1,0,3,2]
+        v = op(v, dpp_d<0x4E>(v));  // quad_perm [2,3,0,1]
+        if constexpr (kBW == 8) {
+            v = op(v, dpp_d<0x141>(v));  // row_half_mirror
+        } else {
+            static_assert(kBW == 8 || kBW == 16, "8 or 16 waves");
+            v = op(v, dpp_d<0x124>(v));  // row_ror:4
+            v = op(v, dpp_d<0x128>(v));  // row_ror:8
+        }
+        g0 = lane_d(v, 0);
+        g1 = lane_d(v, kBW);
+    };
+
+    // Reduce-barrier: the totals of acc0 (sum) and acc1 (sum, or maximum).  ONE: in every thread; else in
+    // wave 0, with `mid` run by waves 1.. once the workgroup's partials are out.  False in wave 0 (else
+    // ignored) when a wait ran out.
+    auto reduce = [&](unsigned gen, bool max1, double &t0, double &t1, auto mid) -> bool {
+        if constexpr (!ONE && !kTagged) ops_done();  // published rows before the partials
+        const int par = (int)(gen & 1u);
+        if (max1) {
+            const double w0 = wave_reduce_dpp<false>(acc0), w1 = wave_reduce_dpp<true>(acc1);
+            if (lane == 0) {
+                wsum[par][wave] = w0;
+                wsum[par][kBW + wave] = w1;
+            }
+        } else {
+            const double w = wave_sum2(acc0, acc1);
+            if ((lane & 31) == 0) wsum[par][(lane >> 5) * kBW + wave] = w;
+        }
+        __syncthreads();
+        bool ok = true;
+        if constexpr (ONE) {
+            wg_totals(par, max1, t0, t1);
+        } else if (wave == 0) {
+            double g0, g1;
+            wg_totals(par, max1, g0, g1);
+            if (lane < 2) st_coh(a.tagged + ((size_t)par * nwg + bid) * 2 + lane, tag_partial(lane ? g1 : g0, gen));
+            ok = block_poll<BIG ? 2 : 4>(a.tagged, nwg, gen, max1, t0, t1);
+        } else {
+            mid();
+        }
+        return ok;
+    };
+    // scalar state: every thread's (ONE), every lane's of wave 0, or thread 0's in LDS (large instances: registers)
+    constexpr bool kRunLds = !ONE && RPT >= 8;
+    __shared__ CgRun srun;
+    CgRun run;
+    auto fail = [&] {
+        st_coh(&a.ctl->err, 1);
+        s_err = 1;
+    };
+
+    double t0 = 0.0, t1 = 0.0;
+    unsigned pubm = 0;  // bit q: the wave publishes its rows q (the same in all its lanes)
+    // ---- first totals: (r0, r0), max|b| (infinite: some workgroup cannot hold its rows) ----
+    {
+        const bool ok = reduce(0u, true, t0, t1, [] {});
+        if constexpr (ONE) {
+            if (t == 0) bc = Step{t0, t1, 1};
+        } else if (t == 0) {
+            if (!ok) fail();
+            bc = Step{t0, t1, 1};
+        }
+        __syncthreads();
+        if (s_err) return;
+        t0 = bc.alpha;
+        t1 = bc.beta;
+        if constexpr (!ONE) {
+            if (isinf(t1)) {
+                if (bid == 0 && t == 0) a.ctl->zero_all = 1;  // not solved here
+                return;
+            }
+        }
+        if (a.zero_shortcut && t1 == 0.0) {
+            for (int q = 0; q < RPT; ++q) {
+                const int i = block_row<C>(m, bid, (unsigned)(t + q * T));
+                if (i >= 0) a.x[i] = R(0);
+            }
+            if (bid == 0 && t == 0) cg1_init(a.st[0], t0, 1);
+            return;
+        }
+    }
+    // halo slots of this thread
+    const int h0 = t - 64;
+    // BIG: x lies in memory (read and written by its thread of waves 1.. while wave 0 waits for the totals)
+    R *xw = reinterpret_cast<R *>(a.pub) + (size_t)a.nwg * C * (2 * sizeof(typename Pub<R>::Word) / sizeof(R)) + first;
+    if constexpr (BIG) {
+        for (int k = h0; k < C && wave > 0; k += kBF) {
+            const int i = block_row<C>(m, bid, (unsigned)k);
+            xw[k] = i < 0 ? R(0) : a.x[i];
+        }
+    }
+    R hv[ONE || BIG ? 1 : HPT];           // the halo rows' published values (BIG: in LDS)
+    R hs[ONE || BIG ? 1 : HPT];           // their s
+    // position of halo row k of this thread; rows the thread does not have repeat its first one (or position 0)
+    const bool any_halo = h0 >= 0 && h0 < nh;
+    auto halo_pos = [&](int k) {
+        return any_halo ? (unsigned)(ltile[h0 / kTile + k * (kBF / kTile)] * kTile + h0 % kTile) : 0u;
+    };
+    static_assert(kBF % kTile == 0, "a thread's halo rows have the same place in their tiles");
+    constexpr bool kPosReg = !ONE && RPT < 8;
+    unsigned hpos[kPosReg ? HPT : 1];
+    if constexpr (kPosReg) {
+#pragma unroll
+        for (int k = 0; k < HPT; ++k) hpos[k] = halo_pos(k);
+    }
+    // FP32: load until every halo word carries `tag` (bounded); FP64: one load
+    auto fetch_halo = [&](int par, unsigned tag) {
+        if constexpr (!ONE) {
+            // BIG: half of the words at a time (registers)
+            constexpr int HB = BIG ? HPT / 2 : HPT;
+            static_assert(HPT % HB == 0, "whole batches");
+#pragma unroll
+            for (int b = 0; b < HPT; b += HB) {
+                unsigned spins = 0;
+                for (;;) {
+                    typename Pub<R>::Word u[HB];
+#pragma unroll
+                    for (int k = 0; k < HB; ++k)
+                        u[k] = ld_coh(elem(pub.base + (size_t)par * pub.n, kPosReg ? hpos[kPosReg ? b + k : 0] : halo_pos(b + k)));
+                    unsigned stale = 0;
+#pragma unroll
+                    for (int k = 0; k < HB; ++k) {
+                        bool mine = true;
+                        const R got = Pub<R>::open(u[k], tag, mine);
+                        if constexpr (BIG) lps[2 * C + H + h0 + (b + k) * kBF] = got;
+                        else hv[b + k] = got;
+                        stale |= mine ? 0u : 1u;
+                    }
+                    if (!__any(any_halo && stale)) break;
+                    if (++spins > kSpinLimit) {
+                        herr = 1;
+                        break;
+                    }
+                }
+            }
+        }
+    };
+    auto prefetch_halo = [&](int par, unsigned tag) {
+        if constexpr (kTagged) fetch_halo(par, tag);
+    };
+    // w = A r of the own rows (r of the halo rows in LDS), published with `tag`; (r, r) and (r, w)
+    auto product = [&](int par, unsigned tag) {
+        unsigned at = first + (unsigned)t;
+        if constexpr (RPT >= 8) asm volatile("" : "+v"(at));
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) {
+            const int li = t + q * T;
+            const R rv = lr[li];
+            R wv = 0;
+            // large instances: the indices stay packed (hoisted out of the iterations, their unpacked form spills)
+            if constexpr (RPT >= 8) {
+#pragma unroll
+                for (int j = 0; j < NI; ++j) asm volatile("" : "+v"(idx[q][j]));
+            }
+#pragma unroll
+            for (int j = 0; j < NO; ++j) {
+                if (j == NO / 2) wv += dv[q] * rv;
+                const unsigned off = j & 1 ? idx[q][j / 2] >> 16 : idx[q][j / 2] & 0xffffu;
+                wv += val[q][j] * *reinterpret_cast<const R *>(reinterpret_cast<const char *>(lr) + off);
+            }
+            if constexpr (ONE)
+                if (longm >> q & 1u)
+                    for (int e = a.row[li]; e < a.row[li + 1]; ++e)
+                        wv += a.val[a.perm ? a.perm[e] : e] * lr[a.col[e]];
+            if (q < WL) lps[BIG ? 2 * C + 2 * H + li : 0] = wv;
+            else w[q] = wv;
+            if constexpr (!ONE)
+                if (pubm >> q & 1u) {
+                    R out = wv;
+                    if constexpr (RPT >= 8) asm volatile("" : "+v"(out));  // a copy: w is not tied to the word's registers
+                    put_row(par, at + q * T, out, tag);
+                }
+            acc0 += (double)rv * (double)rv;
+            acc1 += (double)wv * (double)rv;
+            if constexpr (RPT >= 8)
+                if (q % 2 == 1) __builtin_amdgcn_sched_barrier(0);  // bounds the loads in flight (registers)
+        }
+    };
+    if constexpr (!ONE) {
+#pragma unroll
+        for (int q = 0; q < RPT; ++q)
+            if (__any(ld_coh(mark + (first + (unsigned)(t + q * T)) / kTile) == a.salt)) pubm |= 1u << q;
+        pubm = (unsigned)__builtin_amdgcn_readfirstlane((int)pubm);
+        if (wave > 0) {
+            fetch_halo(1, 1u);
+#pragma unroll
+            for (int k = 0; k < HPT; ++k) {
+                const int h = h0 + k * kBF;
+                lr[C + h] = BIG ? lps[BIG ? 2 * C + H + h : 0] : hv[BIG ? 0 : k];
+                if constexpr (BIG) lps[2 * C + h] = R(0);
+                else hs[k] = R(0);
+            }
+        }
+        __syncthreads();
+    }
+    // ---- w = A r; gamma = (r, r), delta = (w, r); alpha = gamma / delta ----
+    acc0 = acc1 = 0.0;
+    product(0, 2u);
+    {
+        double g0, g1 = 0.0;
+        const bool ok = reduce(1u, false, g0, g1, [&] { prefetch_halo(0, 2u); });
+        auto start = [&](CgRun &r) {
+            r.rho = g0;
+            r.den = g1;
+            r.alpha = g0 / g1;
+            r.beta = 0.0;
+            r.inv_rho = 1.0 / g0;
+            r.final_res = 0.0;
+            r.active = r.finite = 1;
+            r.converged = 0;
+            r.used = -1;
+        };
+        if constexpr (!kRunLds)
+            if (ONE || wave == 0) start(run);
+        if constexpr (!ONE) {
+            if (t == 0) {
+                if (!ok) fail();
+                if constexpr (kRunLds) start(srun);
+                bc = Step{g0 / g1, 0.0, 1};
+            }
+            __syncthreads();
+            if (s_err) return;
+        }
+    }
+    Step cs;
+    if constexpr (ONE) cs = Step{run.alpha, run.beta, run.active};
+    else cs = bc;
+    for (int it = 0; it < a.maxit && cs.active; ++it) {
+        const R alpha = (R)cs.alpha, beta = (R)cs.beta;
+        acc0 = acc1 = 0.0;
+        // halo rows: the owner's s and r (FP64: w is loaded once the generation that published it is complete)
+        if constexpr (!ONE) {
+            if (wave > 0) {
+                if constexpr (!kTagged) fetch_halo(it & 1, 0u);
+#pragma unroll
+                for (int k = 0; k < HPT; ++k) {
+                    const int h = h0 + k * kBF;
+                    R sh = BIG ? lps[BIG ? 2 * C + h : 0] : hs[BIG ? 0 : k];
+                    sh = fma(beta, sh, BIG ? lps[BIG ? 2 * C + H + h : 0] : hv[BIG ? 0 : k]);
+                    if constexpr (BIG) lps[2 * C + h] = sh;
+                    else hs[k] = sh;
+                    lr[C + h] = fma(-alpha, sh, lr[C + h]);
+                }
+            }
+        }
+        // own rows: p, s, x, r
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) {
+            const int li = t + q * T;
+            const R rv = lr[li];
+            R sm;
+            if constexpr (BIG) {
+                lps[li] = fma(beta, lps[li], rv);
+                sm = fma(beta, lps[C + li], q < WL ? lps[2 * C + 2 * H + li] : w[q]);
+                lps[C + li] = sm;
+            } else {
+                const R pm = fma(beta, p[q], rv);
+                p[q] = pm;
+                x[q] = fma(alpha, pm, x[q]);
+                sm = fma(beta, s[q], w[q]);
+                s[q] = sm;
+            }
+            const R rm = fma(-alpha, sm, rv);
+            lr[li] = rm;
+            if constexpr (RPT >= 8)
+                if (q % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+        }
+        __syncthreads();
+        product((it + 1) & 1, (unsigned)it + 3u);
+        double gam = 0.0, delta = 0.0;
+        const bool ok = reduce((unsigned)it + 2u, false, gam, delta, [&] {
+            if constexpr (BIG) {
+                constexpr int XB = 4;  // rows of x in flight per thread
+                static_assert(!BIG || C % (XB * kBF) == 0, "whole batches");
+                for (int k = h0; k < C; k += XB * kBF) {
+                    R xv[XB];
+#pragma unroll
+                    for (int j = 0; j < XB; ++j) xv[j] = *elem(xw, k + j * kBF);
+#pragma unroll
+                    for (int j = 0; j < XB; ++j) *elem(xw, k + j * kBF) = fma(alpha, lps[k + j * kBF], xv[j]);
+                }
+            }
+            prefetch_halo((it + 1) & 1, (unsigned)it + 3u);
+        });
+        if constexpr (ONE) {
+            block_run_update(a, run, gam, delta, it);
+            cs = Step{run.alpha, run.beta, run.active};
+        } else {
+            if (wave == 0) {
+                if (!ok) {
+                    if (t == 0) fail();
+                } else if constexpr (kRunLds) {
+                    if (t == 0) {
+                        block_run_update(a, srun, gam, delta, it);
+                        bc = Step{srun.alpha, srun.beta, srun.active};
+                    }
+                } else {
+                    block_run_update(a, run, gam, delta, it);
+                    if (t == 0) bc = Step{run.alpha, run.beta, run.active};
+                }
+            }
+            __syncthreads();
+            if (s_err) return;
+            cs = bc;
+        }
+    }
+    if (herr) st_coh(&a.ctl->err, 1);
+    if constexpr (BIG) {
+        for (int k = h0; k < C && wave > 0; k += kBF) {
+            const int i = block_row<C>(m, bid, (unsigned)k);
+            if (i >= 0) a.x[i] = xw[k];
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < (BIG ? 0 : RPT); ++q) {
+        const int li = t + q * T;
+        const int i = block_row<C>(m, bid, (unsigned)li);
+        if (i < 0) continue;
+        a.x[i] = x[q];
+    }
+    if (bid == 0 && t == 0) {
+        auto finish = [&](CgRun &r) {
+            block_run_end(a, r);
+            RhsState st;
+            cg1_init(st, r.rho, 0);
+            st.alpha = r.alpha;
+            st.beta = r.beta;
+            st.final_res = r.final_res;
+            st.active = r.active;
+            st.converged = r.converged;
+            st.finite = r.finite;
+            st.used = r.used;
+            a.st[0] = st;
+        };
+        if constexpr (kRunLds) finish(srun);
+        else finish(run);
+    }
+}
+
+template <typename R, int T, int RPT, int NZ, int HPT, bool BIG, bool ONE>
+__global__ __launch_bounds__(T) void k_cg_block(SolveArgs<R> a) {
+    cg_block<R, T, RPT, NZ, HPT, BIG, ONE>(a, blockIdx.x);
+}
+
+// Batched launch (job lists as for k_cg_local_jobs): systems of up to 2048 rows run the one-workgroup instance that
+// they would run alone, larger ones RPT rows per thread.
+template <typename R, int RPT, int NZ, int HPT>
+__global__ __launch_bounds__(512) void k_cg_block_jobs(const SolveArgs<R> *__restrict__ args,
+                                                       const unsigned *__restrict__ job_off,
+                                                       const unsigned *__restrict__ jobs) {
+    const unsigned j0 = job_off[blockIdx.x], j1 = job_off[blockIdx.x + 1];
+    for (unsigned j = j0; j < j1; ++j) {
+        const unsigned job = (unsigned)__builtin_amdgcn_readfirstlane((int)jobs[j]);
+        const SolveArgs<R> a = args[job >> 16];
+        if (a.n <= 512) cg_block<R, 512, 1, NZ, 1, false, true>(a, 0);
+        else if (a.n <= 1024) cg_block<R, 512, 2, NZ, 1, false, true>(a, 0);
+        else if (a.n <= kBlockJobsOne) cg_block<R, 512, 4, NZ, 1, false, true>(a, 0);
+        else cg_block<R, 512, RPT, NZ, HPT, false, false>(a, job & 0xffffu);
+        __syncthreads();
+    }
+}
+
+// Instances.  One workgroup: up to 1024 threads x 8 rows; several: 512 threads.
+template <typename R, int NZ>
+static BlockKernel one_kernel(long long n) {
+    constexpr bool f32 = sizeof(R) == 4;
+    if (n <= 512) return {(const void *)k_cg_block<R, 512, 1, NZ, 1, false, true>, 512, 1};
+    if (n <= 1024) return {(const void *)k_cg_block<R, 512, 2, NZ, 1, false, true>, 512, 2};
+    if (n <= 2048) return {(const void *)k_cg_block<R, 512, 4, NZ, 1, false, true>, 512, 4};
+    if constexpr (f32) {
+        if (n <= 4096) return {(const void *)k_cg_block<R, 1024, 4, NZ, 1, false, true>, 1024, 4};
+    }
+    return {nullptr, 0, 0};
+}
+template <typename R, int NZ>
+static BlockKernel many_kernel(int rpt) {
+    if constexpr (NZ <= 5) {
+        switch (rpt) {
+            case 1:
+                if constexpr (sizeof(R) == 4) return {(const void *)k_cg_block<R, 512, 1, 5, 2, false, false>, 512, 1};
+                return {nullptr, 0, 0};
+            case 2: return {(const void *)k_cg_block<R, 512, 2, 5, 2, false, false>, 512, 2};
+            case 4: return {(const void *)k_cg_block<R, 512, 4, 5, 3, false, false>, 512, 4};
+            case 8:
+                if constexpr (sizeof(R) == 4) return {(const void *)k_cg_block<R, 512, 8, 5, 4, false, false>, 512, 8};
+                return {nullptr, 0, 0};
+            default: return {nullptr, 0, 0};
+        }
+    } else {
+        switch (rpt) {
+            case 1: return {(const void *)k_cg_block<R, 512, 1, 7, 3, false, false>, 512, 1};
+            case 2: return {(const void *)k_cg_block<R, 512, 2, 7, 4, false, false>, 512, 2};
+            case 4: return {(const void *)k_cg_block<R, 512, 4, 7, 6, false, false>, 512, 4};
+            case 8:
+                if constexpr (sizeof(R) == 4) return {(const void *)k_cg_block<R, 512, 8, 7, 9, false, false>, 512, 8};
+                return {nullptr, 0, 0};
+            case 14:
+                if constexpr (sizeof(R) == 4) return {(const void *)k_cg_block<R, 512, 14, 7, 12, true, false>, 512, 14};
+                return {nullptr, 0, 0};
+            default: return {nullptr, 0, 0};
+        }
+    }
+}
+
+BlockKernel cg_block_one(bool f32, int nz, long long n) {
+    return f32 ? (nz <= 5 ? one_kernel<float, 5>(n) : one_kernel<float, 7>(n))
+               : (nz <= 5 ? one_kernel<double, 5>(n) : one_kernel<double, 7>(n));
+}
+template <typename R, int NZ>
+static BlockKernel jobs_kernel(int rpt) {
+    constexpr int H1 = NZ <= 5 ? 2 : 3, H2 = NZ <= 5 ? 2 : 4, H4 = NZ <= 5 ? 3 : 6;
+    switch (rpt) {
+        case 1: return {(const void *)k_cg_block_jobs<R, 1, NZ, H1>, 512, 1};
+        case 2: return {(const void *)k_cg_block_jobs<R, 2, NZ, H2>, 512, 2};
+        case 4:
+            if constexpr (sizeof(R) == 4 || NZ <= 5) return {(const void *)k_cg_block_jobs<R, 4, NZ, H4>, 512, 4};
+            return {nullptr, 0, 0};
+        case 8:
+            if constexpr (sizeof(R) == 4 && NZ <= 5) return {(const void *)k_cg_block_jobs<R, 8, NZ, 4>, 512, 8};
+            return {nullptr, 0, 0};
+        default: return {nullptr, 0, 0};
+    }
+}
+BlockKernel cg_block_jobs(bool f32, int nz, int rpt) {
+    return f32 ? (nz <= 5 ? jobs_kernel<float, 5>(rpt) : jobs_kernel<float, 7>(rpt))
+               : (nz <= 5 ? jobs_kernel<double, 5>(rpt) : jobs_kernel<double, 7>(rpt));
+}
+BlockKernel cg_block_many(bool f32, int nz, int rpt) {
+    return f32 ? (nz <= 5 ? many_kernel<float, 5>(rpt) : many_kernel<float, 7>(rpt))
+               : (nz <= 5 ? many_kernel<double, 5>(rpt) : many_kernel<double, 7>(rpt));
+}
+
+}  // namespace pict

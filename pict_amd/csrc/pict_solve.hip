@@ -29,82 +29,9 @@
 #include <memory>
 #include <vector>
 
-#include "pict_host.hpp"
-#include "pict_solver.hpp"
+#include "pict_krylov.hpp"
 
 namespace pict {
-
-constexpr int kSolveThreads = 256;
-constexpr int kSlots = 8;              // FP64 partial slots per right-hand side
-constexpr unsigned kSpinLimit = 1u << 23;
-constexpr int kMaxRhs = 4;
-
-// Control block, one 128-byte line per hot word (device memory, zeroed before launch).
-struct Ctl {
-    unsigned count;              // top-level arrivals (one per group)
-    unsigned pad0[31];
-    unsigned gen;                // barrier generation
-    unsigned pad1[31];
-    int err;                     // a wait exceeded its spin limit
-    int zero_all;                // every right-hand side is zero
-    unsigned pad2[30];
-    unsigned group_count[32][32];  // per-group arrivals (a line per group)
-};
-// Resident workgroups (256 threads) per compute unit that a persistent solver grid is sized for.  Grids of seven
-// and eight per unit (1792 and 2048 workgroups: the 1.77 M-row channel pressure system on the lean grid-wide CG
-// and on the textbook CG) ended at the barrier's spin limit.  They sat exactly at the occupancy query's maximum,
-// which SGPRs set for those kernels (102-106 per wave: 7 waves per SIMD), while grids at a VGPR-set maximum run;
-// the counters and the spin budget do not depend on the grid size.  Four per unit stays below the SGPR limit of
-// every solver kernel; kernels whose VGPRs allow fewer take the query's figure.
-constexpr int kMaxResidentWgsPerCu = 4;
-constexpr int kGroups = 8;       // arrival tree fan-in (one group per XCD when blocks are dealt round-robin)
-
-// Loads and stores that one workgroup uses to exchange data with another: agent-scope atomic
-// operations (sc1 on gfx950), coherent across the XCDs' L2 caches without L2 writeback or
-// invalidation.
-template <typename T>
-__device__ __forceinline__ void st_coh(T *p, T v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename T>
-__device__ __forceinline__ T ld_coh(const T *p) {
-    return __hip_atomic_load(const_cast<T *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// wait until every memory operation this thread issued has completed
-__device__ __forceinline__ void ops_done() {
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    __builtin_amdgcn_s_waitcnt(0);
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-}
-
-struct RhsState {
-    double rho, rho_prev, alpha, omega, beta;
-    double best_crit, last_crit;
-    int active, converged, finite, used;
-    int best_it, rising, save_best, restore_best;
-    double final_res;
-    double pad;
-};
-
-template <typename R>
-struct SolveArgs {
-    const int32_t *row, *col, *perm;  // perm != nullptr: use A^T (value of (j,i) for entry (i,j))
-    const R *val;
-    const R *b;
-    R *x;
-    R *r, *rhat, *p0, *p1, *v0, *v1, *s, *t, *best;  // each [nrhs*n]
-    double *partials;                              // partial_doubles(nwg) (grid-wide kernels)
-    Ctl *ctl;
-    RhsState *st;                                  // [nrhs]
-    int n, nrhs, maxit, conv, reset_steps, return_best, zero_shortcut;
-    double tol;
-    unsigned nwg;
-    double crit_scale;                             // criterion factor: 1/sqrt(n) (NORM2_NORMALIZED), 1/n (ABS_MEAN), 1
-    unsigned long long *tagged;                    // tagged partials [2][nwg][kSlots], zeroed (k_cg_local packs its
-                                                   // NS values per workgroup: [2][nwg][NS])
-    void *pub;                                     // k_cg_local: published rows r, w, s [3][2][n], zeroed
-    int salt;                                      // k_cg_local: stamp of this launch's foreign-read marks
-};
 
 // --------------------------------------------------------------------------
 // workgroup reductions (wave64 shuffles + LDS), results broadcast to all lanes
@@ -202,9 +129,6 @@ __device__ __forceinline__ void wait_gen(Ctl *ctl, unsigned my_gen, int &s_err) 
     }
     __syncthreads();
 }
-
-// slot layout of the partial sums (per workgroup and right-hand side)
-enum { S_RR = 0, S_ASUM = 1, S_AMAX = 2, S_D0 = 3, S_D1 = 4, S_BMAX = 5 };
 
 // Flush NS accumulators per RHS of this thread: workgroup-reduce and store
 // this workgroup's partials for the slots `ids`.
@@ -312,30 +236,6 @@ __device__ __forceinline__ void acc_res(double (&acc)[NR][NS], int k, R rv) {
 constexpr int kPartStride = kMaxRhs * kSlots;
 constexpr int kTreeGroups = 32;
 constexpr size_t partial_doubles(long long nwg) { return ((size_t)2 * (size_t)nwg + kTreeGroups + 1) * kPartStride; }
-
-// Wave64 reductions in DPP (quad and row rotations within 16-lane rows, then the
-// four row totals in a fixed order): every lane of the wave gets the same total,
-// and the result depends only on the inputs, so every workgroup reducing the same
-// values gets bitwise the same result.
-template <int CTRL>
-__device__ __forceinline__ double dpp_d(double v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, false);
-    return __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ double lane_d(double v, int lane) {
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
-                            __builtin_amdgcn_readlane(__double2loint(v), lane));
-}
-template <bool MAX>
-__device__ __forceinline__ double wave_reduce_dpp(double v) {
-    auto op = [](double x, double y) { return MAX ? fmax(x, y) : x + y; };
-    v = op(v, dpp_d<0xB1>(v));   // quad_perm [1,0,3,2]
-    v = op(v, dpp_d<0x4E>(v));   // quad_perm [2,3,0,1]
-    v = op(v, dpp_d<0x124>(v));  // row_ror:4
-    v = op(v, dpp_d<0x128>(v));  // row_ror:8
-    return op(op(lane_d(v, 0), lane_d(v, 16)), op(lane_d(v, 32), lane_d(v, 48)));
-}
 
 // FENCE = false: the caller exchanges its vectors with agent-scope atomics (st_coh / ld_coh); every wave
 // waits for its stores before the workgroup arrives, the barrier's own data go the same way, and no L2
@@ -757,25 +657,6 @@ __device__ __forceinline__ void cg1_update(const SolveArgs<R> &a, RhsState &st, 
     st.rho = gam;
 }
 
-// first reduction of a solve: rho = (r0, r0); zero-RHS shortcut flag in omega
-__device__ __forceinline__ void cg1_init(RhsState &st, double rr, int zero_all) {
-    st.rho = rr;
-    st.alpha = 0;
-    st.beta = 0;
-    st.omega = zero_all;
-    st.active = zero_all ? 0 : 1;
-    st.converged = zero_all;
-    st.finite = 1;
-    st.used = -1;
-    st.final_res = 0;
-    st.best_crit = 0;
-    st.last_crit = 0;
-    st.best_it = -1;
-    st.rising = 0;
-    st.save_best = 0;
-    st.restore_best = 0;
-}
-
 // ==========================================================================
 // CG, single-reduction form (Chronopoulos & Gear 1989): the same Krylov
 // iterates as cgSolveGPU (cg_solver_kernel.cu:114-456) in exact arithmetic,
@@ -794,6 +675,7 @@ __device__ __forceinline__ void cg1_init(RhsState &st, double rr, int zero_all) 
 // ==========================================================================
 template <typename R, int NRHS, bool LEAN>
 __global__ __launch_bounds__(kSolveThreads) void k_cg1(SolveArgs<R> a) {
+    if (a.gate && *a.gate == 0) return;
     __shared__ double red[NRHS * kSlots];
     __shared__ RhsState sst[NRHS];
     __shared__ int s_err;
@@ -1165,107 +1047,12 @@ __global__ __launch_bounds__(kSolveThreads) void k_cg1(SolveArgs<R> a) {
 // Both regions are zeroed before the launch (tag 0 is never awaited).
 // ==========================================================================
 
-typedef unsigned long long u64;
-// A slot is rewritten every second generation, so a stale slot is exactly two generations
-// old: (generation + 1) mod 4 tells them apart, and the zeroed start (tag 0) is not awaited
-// before every slot has been written once.
-__device__ __forceinline__ u64 tag_partial(double v, unsigned gen) {
-    return (__double_as_longlong(v) & ~3ull) | (u64)((gen + 1u) & 3u);
-}
-__device__ __forceinline__ bool partial_ready(u64 u, unsigned gen) { return (unsigned)(u & 3u) == ((gen + 1u) & 3u); }
-__device__ __forceinline__ double partial_value(u64 u) { return __longlong_as_double((long long)(u & ~3ull)); }
-
-// Published row values of one vector: [2][n] (parity), FP32 as (value, tag) words.
-template <typename R>
-struct Pub;
-template <>
-struct Pub<float> {
-    u64 *base;
-    int n;
-    __device__ __forceinline__ void put(int par, int i, float v, unsigned tag) const {
-        st_coh(base + (size_t)par * n + i, ((u64)tag << 32) | (u64)__float_as_uint(v));
-    }
-    // value of row c (parity par) once it carries `tag`; NaN after a bounded wait
-    __device__ __forceinline__ float get(int par, int c, unsigned tag, int &err) const {
-        if (err) return __int_as_float(0x7fc00000);
-        const u64 *p = base + (size_t)par * n + c;
-        u64 u = ld_coh(p);
-        unsigned spins = 0;
-        while ((unsigned)(u >> 32) != tag) {
-            if (++spins > kSpinLimit) {
-                err = 1;
-                return __int_as_float(0x7fc00000);
-            }
-            u = ld_coh(p);
-        }
-        return __uint_as_float((unsigned)u);
-    }
-    // raw word of row c (one load, no wait), then its value and whether it carries `tag`
-    using Word = u64;
-    __device__ __forceinline__ u64 word(int par, int c) const { return ld_coh(base + (size_t)par * n + c); }
-    static __device__ __forceinline__ float open(u64 u, unsigned tag, bool &ok) {
-        ok = ok & ((unsigned)(u >> 32) == tag);
-        return __uint_as_float((unsigned)u);
-    }
-    static constexpr bool kTagged = true;
-};
-template <>
-struct Pub<double> {
-    double *base;
-    int n;
-    __device__ __forceinline__ void put(int par, int i, double v, unsigned) const {
-        st_coh(base + (size_t)par * n + i, v);
-    }
-    __device__ __forceinline__ double get(int par, int c, unsigned, int &) const {
-        return ld_coh(base + (size_t)par * n + c);
-    }
-    using Word = double;
-    __device__ __forceinline__ double word(int par, int c) const { return ld_coh(base + (size_t)par * n + c); }
-    static __device__ __forceinline__ double open(double u, unsigned, bool &) { return u; }
-    static constexpr bool kTagged = false;
-};
-
 // Reduce-barrier on tagged partials: the workgroup's totals of acc go to its line of
 // the generation's set (tagged); wave 0 then reads all nwg lines until every slot
 // carries the generation's tag and reduces them in a fixed order (red[ids[s]], thread
 // 0's view).  The two sets alternate by generation parity: a set is written again
 // only after every workgroup has passed the next generation.  `wait_rows`: the
 // workgroup's row stores must complete before its partials go out (untagged rows).
-// Reduction layouts of k_cg_local (slot ids and whether a slot is a maximum), as types so
-// that every use folds to constants.  With a norm-2 criterion only (r,r) and (w,r) (and
-// max|b| in the first pass) are needed; the sum and the maximum of |r| only for the
-// absolute criteria.
-struct CgFirstFull {
-    static constexpr int NS = 4;
-    static constexpr int ID[4] = {S_RR, S_ASUM, S_AMAX, S_BMAX};
-    static constexpr bool MAX[4] = {false, false, true, true};
-};
-struct CgIterFull {
-    static constexpr int NS = 4;
-    static constexpr int ID[4] = {S_RR, S_ASUM, S_AMAX, S_D0};
-    static constexpr bool MAX[4] = {false, false, true, false};
-};
-struct CgFirst {
-    static constexpr int NS = 2;
-    static constexpr int ID[2] = {S_RR, S_BMAX};
-    static constexpr bool MAX[2] = {false, true};
-};
-struct CgIter {
-    static constexpr int NS = 2;
-    static constexpr int ID[2] = {S_RR, S_D0};
-    static constexpr bool MAX[2] = {false, false};
-};
-template <bool FULL>
-struct CgSlots {
-    using First = CgFirstFull;
-    using Iter = CgIterFull;
-};
-template <>
-struct CgSlots<false> {
-    using First = CgFirst;
-    using Iter = CgIter;
-};
-
 // FILL: the workgroup writes every slot of its line (unused ones as 0), for callers whose layouts differ from
 // one generation to the next: each slot is then rewritten every second generation, which the 2-bit tag needs
 // to tell a stale slot from a current one.
@@ -1440,66 +1227,6 @@ __device__ __forceinline__ bool packed_poll(const u64 *part, unsigned nwg, unsig
 #pragma unroll
     for (int s = 0; s < NS; ++s) t[L::ID[s]] = L::MAX[s] ? wave_reduce_dpp<true>(v[s]) : wave_reduce_dpp<false>(v[s]);
     return true;
-}
-
-// 1/d to about one ulp: the hardware estimate and two Newton steps
-__device__ __forceinline__ double rcp64(double d) {
-    double y = __builtin_amdgcn_rcp(d);
-    double e = fma(-d, y, 1.0);
-    y = fma(y, e, y);
-    e = fma(-d, y, 1.0);
-    return fma(y, e, y);
-}
-
-// Solver state of k_cg_local's iterations, held by every lane of wave 0 (all lanes compute the
-// same values from the same totals).
-struct CgRun {
-    double rho, inv_rho, den, alpha, beta;  // alpha = rho / den
-    double best_crit, last_crit, final_res;
-    int active, converged, finite, used, best_it, rising, save_best, restore_best;
-};
-
-// cg1_update in the form k_cg_local runs it: the same tests (convergence cg_solver_kernel.cu:306-313,
-// best result :330-346), and the next step from
-//   beta' = gamma' / rho,  delta' - beta' gamma' / alpha = delta' - beta'^2 den,  alpha' = gamma' / that,
-// equal to cg1_update's alpha' and beta' in exact arithmetic.  The candidates are formed before the
-// tests, so one reciprocal (not three dependent divisions) lies on the path to the next iteration.
-template <bool FULL, typename R>
-__device__ __forceinline__ void cg_run_update(const SolveArgs<R> &a, CgRun &st, const double (&t)[kSlots], int it) {
-    const double gam = t[S_RR];
-    const double beta_n = gam * st.inv_rho;
-    const double den_n = fma(-beta_n * beta_n, st.den, t[S_D0]);
-    const double alpha_n = gam * rcp64(den_n);
-    const double inv_rho_n = rcp64(gam);
-    double crit = sqrt(gam) * a.crit_scale;
-    if constexpr (FULL)
-        crit = (a.conv == PICT_CONV_NORM2 || a.conv == PICT_CONV_NORM2_NORMALIZED) ? crit
-               : a.conv == PICT_CONV_ABS_MAX                                      ? t[S_AMAX]
-                                                                                  : t[S_ASUM] * a.crit_scale;
-    st.save_best = 0;
-    if (!isfinite(crit)) {
-        st.converged = 0; st.used = it; st.final_res = crit; st.finite = 0; st.active = 0;
-        return;
-    }
-    if (a.return_best) {
-        if (it == 0 || crit < st.best_crit) { st.best_crit = crit; st.best_it = it; st.save_best = 1; }
-        if (it > 0 && crit >= st.last_crit) ++st.rising; else st.rising = 0;
-        st.last_crit = crit;
-    }
-    st.used = it;
-    st.final_res = crit;
-    if (crit < a.tol) { st.converged = 1; st.finite = 1; st.active = 0; return; }
-    if (a.return_best && (it == a.maxit - 1 || st.rising >= 100)) {
-        st.restore_best = st.best_it != it;
-        st.converged = 0; st.used = st.best_it; st.final_res = st.best_crit; st.finite = 1;
-        st.active = 0;
-        return;
-    }
-    st.alpha = alpha_n;
-    st.beta = beta_n;
-    st.den = den_n;
-    st.rho = gam;
-    st.inv_rho = inv_rho_n;
 }
 
 // Foreign entries (columns owned by another workgroup) of a thread's rows: at most NH per
@@ -1937,6 +1664,7 @@ __device__ __forceinline__ void cg_local(const SolveArgs<R> &a, unsigned bid) {
 
 template <typename R, int RPT, int NZ, bool FULL>
 __global__ __launch_bounds__(kSolveThreads) void k_cg_local(SolveArgs<R> a) {
+    if (a.gate && *a.gate == 0) return;
     cg_local<R, RPT, NZ, FULL>(a, blockIdx.x);
 }
 
@@ -1952,6 +1680,7 @@ __global__ __launch_bounds__(kSolveThreads) void k_cg_local_jobs(const SolveArgs
     for (unsigned j = j0; j < j1; ++j) {
         const unsigned job = jobs[j];
         const SolveArgs<R> a = args[job >> 16];
+        if (a.gate && *a.gate == 0) continue;  // solved by k_cg_block_jobs
         cg_local<R, RPT, NZ, FULL>(a, job & 0xffffu);
         __syncthreads();
     }
@@ -2450,9 +2179,11 @@ __global__ void k_solve_out(const RhsState *st, int nrhs, const int *err, RhsSta
     if (k == 0) *err_out = *err;
 }
 
-// zero n 64-bit words (the tagged regions of k_cg_local, before its launch)
-__global__ void k_zero64(u64 *p, size_t n) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = 0;
+// zero n (and m) 64-bit words (control block and tagged regions, before a solver kernel's launch)
+__global__ void k_zero64(u64 *p, size_t n, u64 *p2, size_t m) {
+    const size_t step = (size_t)gridDim.x * blockDim.x, i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    for (size_t i = i0; i < n; i += step) p[i] = 0;
+    for (size_t i = i0; i < m; i += step) p2[i] = 0;
 }
 
 // ==========================================================================
@@ -2763,7 +2494,7 @@ thread_local hipEvent_t g_ev[2] = {nullptr, nullptr};
 
 // Occupancy (resident workgroups per CU) of a solver kernel on the current device, cached, at most
 // kMaxResidentWgsPerCu: every workgroup of a persistent solver grid has to be resident at once.
-pict_status occupancy(const void *kernel, int &occ, int &cus) {
+pict_status occupancy(const void *kernel, int &occ, int &cus, int threads = kSolveThreads) {
     struct Entry { int dev; const void *k; int occ; int cus; };
     static thread_local std::vector<Entry> cache;
     int dev;
@@ -2775,8 +2506,8 @@ pict_status occupancy(const void *kernel, int &occ, int &cus) {
             return PICT_OK;
         }
     PICT_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    PICT_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, kSolveThreads, 0));
-    if (occ > kMaxResidentWgsPerCu) occ = kMaxResidentWgsPerCu;
+    PICT_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, threads, 0));
+    occ = std::min(occ, kMaxResidentWgsPerCu * kSolveThreads / threads);
     cache.push_back({dev, kernel, occ, cus});
     return PICT_OK;
 }
@@ -2894,10 +2625,71 @@ struct Plan {
     bool full;      // k_cg_local reduces the sum and maximum of |r| too
     bool lean;      // k_cg1 without the register row cache
     int cus;        // compute units of the device
+    // k_cg_block in front (null: none); unless it runs on one workgroup, the kernel above is queued behind it for
+    // the systems it cannot hold
+    BlockKernel block;
+    bool block_one;
+    int block_nz;
+    long long block_nwg;
 };
 
+// Workgroups of k_cg_block for n rows, C rows each: as many as the rows fill; 3-D systems (7-entry rows) leave room
+// for blocks of whole grid lines.
+long long block_wgs(long long n, long long C, int nz) { return ((nz <= 5 ? n : n * 17 / 10) + C - 1) / C; }
+
+// Bytes of k_cg_block's regions (the marks, one per tile of 8 rows, then from `off` the tagged partials and published
+// rows, zeroed before a launch) for nwg workgroups of C rows.
+size_t block_region(long long nwg, long long C, size_t &off) {
+    const size_t pos = (size_t)nwg * C;
+    off = (pos / 8 * sizeof(int) + 255) & ~size_t(255);
+    return 8 * ((size_t)nwg * 4 + 2 * pos);
+}
+
+// k_cg_block's shape for a system: instance and workgroups, or none (a longer row on average than its registers take,
+// or more rows than fit on the chip).  Measured per iteration, FP32 unless said, before = the kernel of plan_general:
+//  - up to 4096 rows (FP64: 2048) one workgroup, whose iteration has no trip through memory: 32 x 32 cavity 2.0 -> 0.62
+//    us, 64 x 64 2.26 -> 1.28 (on several workgroups 1.4 and 1.7); beyond, the rows per compute unit cost more than the
+//    barrier saves (80 x 80: 2.6 on one, 1.85 on 13).
+//  - 5-entry rows: one row per thread up to 64 workgroups, two up to 128 (256 x 256: 2.73 -> 1.8, the same on 64 and
+//    128 workgroups, 2.1 on 32 with four rows, 2.9 with eight); then four and eight as far as the compute units reach
+//    (640 x 500: 13.3 -> 3.0).  FP64 words carry no tag, so their exchange is not hidden and the gain small: two rows
+//    per thread from the start (97 x 61: 2.8 -> 2.4, 320 x 256: 3.8 -> 3.5, 200 x 150: 3.0 both).
+//  - 7-entry rows: the barrier grows past 128 workgroups (57 x 35 x 30: 2.6 on 199 with one row per thread, 1.95 on 99
+//    with two, 2.1 on 50 with four; before: 4.2), a row costs 0.25 us (131 x 67 x 45: 3.1 with four rows, 4.1 with
+//    eight; before: 17.2); 150 x 90 x 60: 25 -> 5.4, 192 x 96 x 96 with fourteen: 40 -> 7.8.
+// PICT_CG_LOCAL_WGS (a workgroup budget of k_cg_local) selects plan_general's kernels.
 template <typename R>
-pict_status plan_solve(const pict_csr_desc *A, int nrhs, const pict_solve_opts *o, Plan &pl) {
+void plan_block(const pict_csr_desc *A, int cus, Plan &pl) {
+    const long long n = A->n;
+    if ((long long)A->nnz > 7 * n || getenv("PICT_CG_LOCAL_WGS")) return;
+    const bool f32 = sizeof(R) == 4;
+    const int nz = (long long)A->nnz <= 5 * n ? 5 : 7;
+    pl.block_nz = nz;
+    pl.block = cg_block_one(f32, nz, n);
+    pl.block_one = pl.block.kernel != nullptr;
+    pl.block_nwg = 1;
+    if (pl.block_one) return;
+    const long long cap = std::min(cus, 256);
+    for (int rpt : {1, 2, 4, 8, 14}) {
+        const BlockKernel k = cg_block_many(f32, nz, rpt);
+        if (!k.kernel) continue;  // (also FP64 5-entry rows, one per thread)
+        const long long C = (long long)k.threads * rpt;
+        long long nwg = block_wgs(n, C, nz);
+        const long long limit = rpt > 2 ? cap : std::min<long long>(cap, nz <= 5 && rpt == 1 ? 64 : 128);
+        if (nz > 5 && rpt > 2) {
+            // blocks of whole lines rarely fill a workgroup: a margin, except for the last instance
+            if (n > (rpt == 14 ? cap * C : cap * C * 85 / 100)) continue;
+            nwg = std::min(nwg, cap);
+        }
+        if (nwg > limit) continue;
+        pl.block = k;
+        pl.block_nwg = nwg;
+        return;
+    }
+}
+
+template <typename R>
+pict_status plan_general(const pict_csr_desc *A, int nrhs, const pict_solve_opts *o, Plan &pl) {
     const int n = A->n;
     // PICT_CG_TEXTBOOK=1 selects the two-barrier textbook CG kernel (diagnostics / parity checks)
     const char *tb_env = getenv("PICT_CG_TEXTBOOK");
@@ -3008,23 +2800,44 @@ pict_status plan_solve(const pict_csr_desc *A, int nrhs, const pict_solve_opts *
     return PICT_OK;
 }
 
+template <typename R>
+pict_status plan_solve(const pict_csr_desc *A, int nrhs, const pict_solve_opts *o, Plan &pl) {
+    pict_status st = plan_general<R>(A, nrhs, o, pl);
+    if (st) return st;
+    if (pl.kind == Kind::kCG1 && nrhs == 1 && o->residual_reset_steps <= 0 && !o->return_best_result &&
+        (o->convergence_criterion == PICT_CONV_NORM2 || o->convergence_criterion == PICT_CONV_NORM2_NORMALIZED))
+        plan_block<R>(A, pl.cus, pl);
+    return PICT_OK;
+}
+
 // Workspace of one solve: vectors | FP64 partials | final states | transpose map | control block |
 // k_cg_local's tagged partials and published rows.  The control block and the regions after it
-// are zeroed by one fill kernel before the launch.
+// are zeroed by one fill kernel before the launch.  k_cg_block's marks, tagged partials and published rows lie in
+// the vectors, which the general kernel only writes after k_cg_block has left the system to it (block_extra: bytes
+// they need beyond the vectors).
 struct Layout {
     size_t vec, off_part, off_st, off_perm, off_ctl, off_zero, words_tagged, words_zero, total;
+    size_t off_block, block_words;  // k_cg_block: tagged partials and published rows
 };
 
 template <typename R>
 Layout layout_of(const pict_csr_desc *A, int nrhs, const pict_solve_opts *o, const Plan &pl) {
     auto al = [](size_t b) { return (b + 255) & ~size_t(255); };
-    Layout L;
+    Layout L{};
     const size_t n = (size_t)A->n;
     L.vec = n * nrhs;
     const int nvec = pl.kind == Kind::kCGTextbook ? (o->return_best_result ? 5 : 4) : 9;
     const size_t bytes_part = sizeof(double) * partial_doubles(pl.nwg);
     const size_t bytes_perm = (o->transpose_a && !A->transpose_perm) ? sizeof(int32_t) * (size_t)A->nnz : 0;
-    L.off_part = al(sizeof(R) * L.vec * nvec);
+    size_t bytes_vec = sizeof(R) * L.vec * nvec;
+    if (pl.block.kernel) {
+        const long long C = (long long)pl.block.threads * pl.block.rpt;
+        const size_t bytes = pl.block_one ? 0 : block_region(pl.block_nwg, C, L.off_block);
+        L.block_words = bytes / 8;
+        // (the large instances keep x behind)
+        bytes_vec = std::max<size_t>(bytes_vec, L.off_block + bytes + sizeof(R) * (size_t)(pl.block_nwg * C));
+    }
+    L.off_part = al(bytes_vec);
     L.off_st = L.off_part + al(bytes_part);
     L.off_perm = L.off_st + al(sizeof(RhsState) * nrhs);
     L.off_ctl = L.off_perm + al(bytes_perm);
@@ -3048,7 +2861,11 @@ pict_status enqueue_typed(const pict_csr_desc *A, const void *rhs, void *x, int 
     const Kind kind = pl.kind;
     const void *kernel = pl.kernel;
     const long long nwg = pl.nwg;
-    const Layout L = layout_of<R>(A, nrhs, o, pl);
+    Layout L = layout_of<R>(A, nrhs, o, pl);
+    if (ws_in && ws_bytes < L.total && pl.block.kernel) {  // a caller's workspace without room for k_cg_block
+        pl.block.kernel = nullptr;
+        L = layout_of<R>(A, nrhs, o, pl);
+    }
     const size_t vec = L.vec;
 
     char *ws = (char *)ws_in;
@@ -3107,8 +2924,9 @@ pict_status enqueue_typed(const pict_csr_desc *A, const void *rhs, void *x, int 
     {
         // control block (+ k_cg_local's tagged regions): a fill kernel, which a captured graph replays safely
         const size_t words = (off_zero - off_ctl) / 8 + L.words_zero;
-        const unsigned blocks = (unsigned)std::min<size_t>((words + 255) / 256, 1024);
-        hipLaunchKernelGGL(k_zero64, dim3(blocks), dim3(256), 0, stream, (unsigned long long *)(ws + off_ctl), words);
+        const unsigned blocks = (unsigned)std::min<size_t>((words + L.block_words + 255) / 256, 1024);
+        hipLaunchKernelGGL(k_zero64, dim3(blocks), dim3(256), 0, stream, (unsigned long long *)(ws + off_ctl), words,
+                           (u64 *)(ws + L.off_block), pl.block.kernel ? L.block_words : (size_t)0);
         PICT_HIP_TRY(hipGetLastError());
     }
     if (o->transpose_a && A->transpose_perm) {
@@ -3130,7 +2948,20 @@ pict_status enqueue_typed(const pict_csr_desc *A, const void *rhs, void *x, int 
     }
     void *args[] = {&a};
     if (ev0) PICT_HIP_TRY(hipEventRecord(ev0, stream));
-    if (plain_launch_enabled() && nwg <= pl.cus)
+    if (pl.block.kernel) {
+        SolveArgs<R> ba = a;
+        ba.p0 = (R *)ws;
+        ba.tagged = (unsigned long long *)(ws + L.off_block);
+        ba.pub = ba.tagged + (size_t)pl.block_nwg * 4;
+        ba.nwg = (unsigned)pl.block_nwg;
+        void *bargs[] = {&ba};
+        PICT_HIP_TRY(hipLaunchKernel(pl.block.kernel, dim3((unsigned)pl.block_nwg), dim3(pl.block.threads), bargs, 0,
+                                     stream));
+        a.gate = &a.ctl->zero_all;
+    }
+    if (pl.block.kernel && pl.block_one)
+        ;
+    else if (plain_launch_enabled() && nwg <= pl.cus)
         PICT_HIP_TRY(hipLaunchKernel(kernel, dim3((unsigned)nwg), dim3(kSolveThreads), args, 0, stream));
     else
         PICT_HIP_TRY(hipLaunchCooperativeKernel(kernel, dim3((unsigned)nwg), dim3(kSolveThreads), args, 0, stream));
@@ -3230,6 +3061,15 @@ struct BatchSolve {
     std::vector<char> args_host;
     std::vector<unsigned> job_off, jobs;
     double makespan = 0.0;
+    // k_cg_block_jobs in front (null: none) with its own workgroups, lists and argument table; the kernel above is
+    // queued behind it for the systems it cannot hold
+    const void *block = nullptr;
+    unsigned block_grid = 0;
+    bool coop = true;  // the general kernel is a cooperative launch
+    std::vector<int> block_nwg;
+    size_t off_bargs = 0, off_bjoboff = 0, off_bjobs = 0;
+    std::vector<char> bargs_host;
+    std::vector<unsigned> bjob_off, bjobs;
     ~BatchSolve() {
         if (arena) (void)hipFree(arena);
     }
@@ -3287,19 +3127,20 @@ __global__ __launch_bounds__(256) void k_batch_err(const SolveArgs<R> *args, int
     if (threadIdx.x == 0) *out = any;
 }
 
-// List scheduling of the systems' jobs onto b.grid workgroups (cost: estimated time of each solve).
-void schedule(BatchSolve &b, const std::vector<double> &cost) {
-    const unsigned G = b.grid;
-    std::vector<int> order(b.count);
-    for (int s = 0; s < b.count; ++s) order[s] = s;
+// List scheduling of the systems' jobs onto `grid` workgroups (cost: estimated time of each solve); returns the
+// makespan.
+double schedule(int count, const std::vector<int> &nwg, unsigned grid, const std::vector<double> &cost,
+                std::vector<unsigned> &job_off, std::vector<unsigned> &jobs) {
+    std::vector<int> order(count);
+    for (int s = 0; s < count; ++s) order[s] = s;
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cost[x] > cost[y]; });
-    std::vector<double> avail(G, 0.0);
-    std::vector<std::vector<unsigned>> lists(G);
-    std::vector<unsigned> idx(G);
-    b.makespan = 0.0;
+    std::vector<double> avail(grid, 0.0);
+    std::vector<std::vector<unsigned>> lists(grid);
+    std::vector<unsigned> idx(grid);
+    double makespan = 0.0;
     for (int s : order) {
-        const unsigned k = (unsigned)b.nwg[s];
-        for (unsigned g = 0; g < G; ++g) idx[g] = g;
+        const unsigned k = (unsigned)nwg[s];
+        for (unsigned g = 0; g < grid; ++g) idx[g] = g;
         auto earlier = [&](unsigned x, unsigned y) { return avail[x] < avail[y] || (avail[x] == avail[y] && x < y); };
         std::nth_element(idx.begin(), idx.begin() + (k - 1), idx.end(), earlier);
         std::sort(idx.begin(), idx.begin() + k);
@@ -3310,15 +3151,39 @@ void schedule(BatchSolve &b, const std::vector<double> &cost) {
             lists[idx[j]].push_back(((unsigned)s << 16) | j);
             avail[idx[j]] = fin;
         }
-        b.makespan = std::max(b.makespan, fin);
+        makespan = std::max(makespan, fin);
     }
-    b.job_off.assign(G + 1, 0);
-    b.jobs.clear();
-    for (unsigned g = 0; g < G; ++g) {
-        b.job_off[g] = (unsigned)b.jobs.size();
-        b.jobs.insert(b.jobs.end(), lists[g].begin(), lists[g].end());
+    job_off.assign(grid + 1, 0);
+    jobs.clear();
+    for (unsigned g = 0; g < grid; ++g) {
+        job_off[g] = (unsigned)jobs.size();
+        jobs.insert(jobs.end(), lists[g].begin(), lists[g].end());
     }
-    b.job_off[G] = (unsigned)b.jobs.size();
+    job_off[grid] = (unsigned)jobs.size();
+    return makespan;
+}
+void schedule(BatchSolve &b, const std::vector<double> &cost) {
+    b.makespan = schedule(b.count, b.nwg, b.grid, cost, b.job_off, b.jobs);
+    if (b.block) b.makespan = schedule(b.count, b.block_nwg, b.block_grid, cost, b.bjob_off, b.bjobs);
+}
+// the argument and job tables to the device, in stream order
+pict_status upload_jobs(const BatchSolve &b, hipStream_t stream) {
+    auto put = [&](size_t off, const std::vector<unsigned> &v) {
+        return v.empty() ? hipSuccess
+                         : hipMemcpyAsync(b.arena + off, v.data(), sizeof(unsigned) * v.size(), hipMemcpyHostToDevice, stream);
+    };
+    PICT_HIP_TRY(put(b.off_joboff, b.job_off));
+    PICT_HIP_TRY(put(b.off_jobs, b.jobs));
+    PICT_HIP_TRY(put(b.off_bjoboff, b.bjob_off));
+    PICT_HIP_TRY(put(b.off_bjobs, b.bjobs));
+    return PICT_OK;
+}
+pict_status upload_args(const BatchSolve &b, hipStream_t stream) {
+    PICT_HIP_TRY(hipMemcpyAsync(b.arena + b.off_args, b.args_host.data(), b.args_host.size(), hipMemcpyHostToDevice, stream));
+    if (b.block)
+        PICT_HIP_TRY(hipMemcpyAsync(b.arena + b.off_bargs, b.bargs_host.data(), b.bargs_host.size(), hipMemcpyHostToDevice,
+                                    stream));
+    return PICT_OK;
 }
 
 // default schedule estimate: CG iterations grow like the square root of the size (2-D and 3-D
@@ -3334,7 +3199,7 @@ std::vector<double> default_cost(const BatchSolve &b) {
 template <typename R>
 void fill_args(BatchSolve &b, int s, const pict_csr_desc &A, const void *rhs, void *x, const pict_solve_opts *o,
                const std::vector<size_t> &off_vec, const std::vector<size_t> &off_part,
-               const std::vector<size_t> &off_ctl) {
+               const std::vector<size_t> &off_ctl, const std::vector<size_t> &off_blk) {
     auto al = [](size_t v) { return (v + 255) & ~size_t(255); };
     SolveArgs<R> a;
     memset(&a, 0, sizeof a);
@@ -3368,6 +3233,14 @@ void fill_args(BatchSolve &b, int s, const pict_csr_desc &A, const void *rhs, vo
     a.tagged = reinterpret_cast<unsigned long long *>(b.arena + off_ctl[s] + al(sizeof(Ctl)));
     a.pub = a.tagged + (b.local || b.bicg_local ? tagged_words(b.nwg[s]) : 0);
     a.salt = next_salt();
+    if (b.block) {
+        SolveArgs<R> ba = a;  // the marks lie in the vectors (p0)
+        ba.nwg = (unsigned)b.block_nwg[s];
+        ba.tagged = reinterpret_cast<unsigned long long *>(b.arena + off_blk[s]);
+        ba.pub = ba.tagged + (size_t)ba.nwg * 4;
+        memcpy(b.bargs_host.data() + (size_t)s * sizeof ba, &ba, sizeof ba);
+        a.gate = &a.ctl->zero_all;
+    }
     memcpy(b.args_host.data() + (size_t)s * sizeof(SolveArgs<R>), &a, sizeof a);
 }
 
@@ -3441,6 +3314,30 @@ pict_status batch_create_typed(const pict_csr_desc *A, const void *const *rhs, v
         sum += w;
     }
     b->grid = (unsigned)std::min(sum, cap);
+    // k_cg_block_jobs in front, for the same rows per thread, when every system's workgroups can be resident
+    if (b->local && !o->return_best_result && !getenv("PICT_CG_LOCAL_WGS")) {
+        const BlockKernel k = cg_block_jobs(sizeof(R) == 4, b->nz, b->rpt);
+        int bocc = 0, bcus = 0;
+        if (k.kernel && (st = occupancy(k.kernel, bocc, bcus, k.threads))) return st;
+        const long long C = (long long)k.threads * k.rpt, bcap = std::min<long long>((long long)bocc * bcus, 256);
+        bool fits = k.kernel && bocc > 0;
+        long long bsum = 0;
+        b->block_nwg.assign(count, 1);
+        for (int s = 0; s < count && fits; ++s) {
+            if (A[s].n > kBlockJobsOne) b->block_nwg[s] = (int)std::min<long long>(block_wgs(A[s].n, C, b->nz), 65535);
+            fits = b->block_nwg[s] <= bcap && (long long)A[s].nnz <= 7LL * A[s].n;
+            bsum += b->block_nwg[s];
+        }
+        if (fits) {
+            b->block = k.kernel;
+            b->block_grid = (unsigned)std::min<long long>(bsum, (long long)bocc * bcus);
+            b->bargs_host.assign(sizeof(SolveArgs<R>) * count, 0);
+            // the general kernel then usually has nothing to do: one workgroup per compute unit, an ordinary launch
+            b->coop = false;
+            for (int s = 0; s < count; ++s) b->coop = b->coop || b->nwg[s] > cus;
+            if (!b->coop) b->grid = (unsigned)std::min<long long>(sum, cus);
+        }
+    }
     // arena: tables | states | error flag | per-system vectors and partials | per-system control blocks and
     // tagged regions (contiguous: one fill kernel clears them before each launch)
     b->args_stride = sizeof(SolveArgs<R>);
@@ -3451,14 +3348,25 @@ pict_status batch_create_typed(const pict_csr_desc *A, const void *const *rhs, v
     off += al(sizeof(unsigned) * (b->grid + 1));
     b->off_jobs = off;
     off += al(sizeof(unsigned) * (size_t)sum);
+    if (b->block) {
+        size_t bjobs = 0;
+        for (int w : b->block_nwg) bjobs += (size_t)w;
+        b->off_bargs = off;
+        off += al(b->args_stride * count);
+        b->off_bjoboff = off;
+        off += al(sizeof(unsigned) * (b->block_grid + 1));
+        b->off_bjobs = off;
+        off += al(sizeof(unsigned) * bjobs);
+    }
     b->off_states = off;
     off += al(sizeof(RhsState) * (size_t)count * nrhs);
     b->off_err = off;
     off += 256;
-    std::vector<size_t> off_vec(count), off_part(count), off_ctl(count);
+    std::vector<size_t> off_vec(count), off_part(count), off_ctl(count), off_blk(count);
     for (int s = 0; s < count; ++s) {
         off_vec[s] = off;
         off += al(sizeof(R) * (size_t)b->n[s] * nrhs * 9);
+        if (b->block) off += 256;  // (k_cg_block's marks, behind the first vector, round up to whole tiles)
         off_part[s] = off;
         off += al(sizeof(double) * partial_doubles(b->nwg[s]));
     }
@@ -3469,20 +3377,20 @@ pict_status batch_create_typed(const pict_csr_desc *A, const void *const *rhs, v
                              : b->bicg_local ? tagged_words(b->nwg[s]) + 2 * (size_t)nrhs * b->n[s]
                                              : 0;
         off += al(sizeof(Ctl)) + al(sizeof(unsigned long long) * words);
+        if (b->block) {
+            size_t marks = 0;
+            off_blk[s] = off;
+            if (b->n[s] > kBlockJobsOne) off += al(block_region(b->block_nwg[s], 512LL * b->rpt, marks));
+        }
     }
     b->zero_words = (off - b->off_zero) / sizeof(unsigned long long);
     b->total = off;
     PICT_HIP_TRY(hipMalloc((void **)&b->arena, b->total));
     b->args_host.assign(b->args_stride * count, 0);
-    for (int s = 0; s < count; ++s) fill_args<R>(*b, s, A[s], rhs[s], x[s], o, off_vec, off_part, off_ctl);
+    for (int s = 0; s < count; ++s) fill_args<R>(*b, s, A[s], rhs[s], x[s], o, off_vec, off_part, off_ctl, off_blk);
     std::vector<double> c = cost ? std::vector<double>(cost, cost + count) : default_cost(*b);
     schedule(*b, c);
-    PICT_HIP_TRY(hipMemcpyAsync(b->arena + b->off_args, b->args_host.data(), b->args_host.size(),
-                                hipMemcpyHostToDevice, stream));
-    PICT_HIP_TRY(hipMemcpyAsync(b->arena + b->off_joboff, b->job_off.data(), sizeof(unsigned) * b->job_off.size(),
-                                hipMemcpyHostToDevice, stream));
-    PICT_HIP_TRY(hipMemcpyAsync(b->arena + b->off_jobs, b->jobs.data(), sizeof(unsigned) * b->jobs.size(),
-                                hipMemcpyHostToDevice, stream));
+    if ((st = upload_args(*b, stream)) || (st = upload_jobs(*b, stream))) return st;
     PICT_HIP_TRY(hipStreamSynchronize(stream));
     *out = b.release();
     return PICT_OK;
@@ -3512,20 +3420,23 @@ pict_status batch_solve_update(BatchSolve *b, const pict_csr_desc *A, const void
                                hipStream_t stream) {
     bool changed = false;
     for (int s = 0; s < b->count; ++s) {
-        char *h = b->args_host.data() + (size_t)s * b->args_stride;
         // the leading members of SolveArgs: row, col, perm, val, b, x
         const void *want[6] = {A[s].row, A[s].index, nullptr, A[s].value, rhs[s], x[s]};
         PICT_CHECK_ARG(A[s].n == b->n[s], "system %d changed size", s);
-        if (memcmp(h, want, sizeof want) != 0) {
-            memcpy(h, want, sizeof want);
-            changed = true;
+        for (std::vector<char> *table : {&b->args_host, &b->bargs_host}) {
+            if (table->empty()) continue;
+            char *h = table->data() + (size_t)s * b->args_stride;
+            if (memcmp(h, want, sizeof want) != 0) {
+                memcpy(h, want, sizeof want);
+                changed = true;
+            }
         }
     }
     if (!changed) return PICT_OK;
     // queued launches read the table: replace it only when they are done
     PICT_HIP_TRY(hipStreamSynchronize(stream));
-    PICT_HIP_TRY(hipMemcpyAsync(b->arena + b->off_args, b->args_host.data(), b->args_host.size(),
-                                hipMemcpyHostToDevice, stream));
+    pict_status st = upload_args(*b, stream);
+    if (st) return st;
     PICT_HIP_TRY(hipStreamSynchronize(stream));
     return PICT_OK;
 }
@@ -3534,10 +3445,8 @@ pict_status batch_solve_reschedule(BatchSolve *b, const double *cost, hipStream_
     std::vector<double> c(cost, cost + b->count);
     schedule(*b, c);
     PICT_HIP_TRY(hipStreamSynchronize(stream));
-    PICT_HIP_TRY(hipMemcpyAsync(b->arena + b->off_joboff, b->job_off.data(), sizeof(unsigned) * b->job_off.size(),
-                                hipMemcpyHostToDevice, stream));
-    PICT_HIP_TRY(hipMemcpyAsync(b->arena + b->off_jobs, b->jobs.data(), sizeof(unsigned) * b->jobs.size(),
-                                hipMemcpyHostToDevice, stream));
+    pict_status st = upload_jobs(*b, stream);
+    if (st) return st;
     PICT_HIP_TRY(hipStreamSynchronize(stream));
     return PICT_OK;
 }
@@ -3547,14 +3456,23 @@ pict_status batch_solve_enqueue(const BatchSolve *b, void *states_out, int *err_
     {
         const unsigned blocks = (unsigned)std::min<size_t>((b->zero_words + 255) / 256, 2048);
         hipLaunchKernelGGL(k_zero64, dim3(blocks ? blocks : 1), dim3(256), 0, stream,
-                           (unsigned long long *)(b->arena + b->off_zero), b->zero_words);
+                           (unsigned long long *)(b->arena + b->off_zero), b->zero_words, (u64 *)nullptr, (size_t)0);
         PICT_HIP_TRY(hipGetLastError());
     }
     void *args_dev = b->arena + b->off_args;
     unsigned *job_off = (unsigned *)(b->arena + b->off_joboff), *jobs = (unsigned *)(b->arena + b->off_jobs);
     void *kargs[] = {&args_dev, &job_off, &jobs};
     if (ev0) PICT_HIP_TRY(hipEventRecord(ev0, stream));
-    PICT_HIP_TRY(hipLaunchCooperativeKernel(b->kernel, dim3(b->grid), dim3(kSolveThreads), kargs, 0, stream));
+    if (b->block) {
+        void *bargs_dev = b->arena + b->off_bargs;
+        unsigned *bjob_off = (unsigned *)(b->arena + b->off_bjoboff), *bjobs = (unsigned *)(b->arena + b->off_bjobs);
+        void *bkargs[] = {&bargs_dev, &bjob_off, &bjobs};
+        PICT_HIP_TRY(hipLaunchCooperativeKernel(b->block, dim3(b->block_grid), dim3(512), bkargs, 0, stream));
+    }
+    if (b->coop)
+        PICT_HIP_TRY(hipLaunchCooperativeKernel(b->kernel, dim3(b->grid), dim3(kSolveThreads), kargs, 0, stream));
+    else
+        PICT_HIP_TRY(hipLaunchKernel(b->kernel, dim3(b->grid), dim3(kSolveThreads), kargs, 0, stream));
     if (ev1) PICT_HIP_TRY(hipEventRecord(ev1, stream));
     int *err = err_out ? err_out : (int *)(b->arena + b->off_err);
     if (b->dtype == PICT_DTYPE_F32)
@@ -3571,14 +3489,17 @@ pict_status batch_solve_enqueue(const BatchSolve *b, void *states_out, int *err_
 }
 
 void batch_solve_describe(const BatchSolve *b, BatchSolveInfo *out) {
-    out->grid = (int)b->grid;
+    out->grid = (int)(b->block ? b->block_grid : b->grid);
     out->rows_per_thread = b->rpt;
     out->rows_per_wg = b->rows_per_wg;
     out->local = b->local || b->bicg_local ? 1 : 0;
-    out->jobs = (int)b->jobs.size();
+    out->jobs = (int)(b->block ? b->bjobs.size() : b->jobs.size());
     out->makespan = b->makespan;
     const bool f32 = b->dtype == PICT_DTYPE_F32;
-    if (b->local)
+    if (b->block)
+        snprintf(out->kernel, sizeof out->kernel, "pict::k_cg_block_jobs<%s, %d, %d>", f32 ? "float" : "double", b->rpt,
+                 b->nz);
+    else if (b->local)
         snprintf(out->kernel, sizeof out->kernel, "pict::k_cg_local_jobs<%s, %d, %d, false>", f32 ? "float" : "double",
                  b->rpt, b->nz);
     else if (b->bicg_local)
@@ -3672,7 +3593,10 @@ pict_status pict_solver_kernel_name(const pict_csr_desc *A, int32_t nrhs, const 
     st = f32 ? plan_solve<float>(A, nrhs, opts, pl) : plan_solve<double>(A, nrhs, opts, pl);
     if (st) return st;
     const int nr = nrhs < kMaxRhs ? nrhs : kMaxRhs;
-    if (pl.local)
+    if (pl.block.kernel)
+        snprintf(buf, (size_t)len, "pict::k_cg_block<%s, %d, %d, %d, %s>", t, pl.block.threads, pl.block.rpt,
+                 pl.block_nz, pl.block_one ? "one" : "several");
+    else if (pl.local)
         snprintf(buf, (size_t)len, "pict::k_cg_local<%s, %d, %d, %s>", t, pl.rpt, pl.nz, pl.full ? "true" : "false");
     else if (pl.bicg_local)
         snprintf(buf, (size_t)len, "pict::k_bicg_local<%d, %d, %d>", pl.rpt, pl.nz, nr);
