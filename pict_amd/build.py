@@ -14,7 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libpict_hip.so")
-SOURCES = ["pict_solve.hip", "pict_stages.hip", "pict_cgblock.hip", "pict_metrics.hip", "pict_grad.hip", "pict_step.hip", "pict_batch.hip", "pict_matvec.hip",
+SOURCES = ["pict_solve.hip", "pict_stages.hip", "pict_cgblock.hip", "pict_bicgblock.hip", "pict_metrics.hip", "pict_grad.hip", "pict_step.hip", "pict_batch.hip", "pict_matvec.hip",
            "pict_noalloc.hip", "pict_sgs.hip", "pict_ilu.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -21,7 +21,7 @@ struct Ctl {
     unsigned gen;                // barrier generation
     unsigned pad1[31];
     int err;                     // a wait exceeded its spin limit
-    int zero_all;                // k_cg: every right-hand side is zero; k_cg_block: the system does not fit it
+    int zero_all;                // k_cg: every right-hand side is zero; k_cg_block, k_bicg_block: the system does not fit
     unsigned pad2[30];
     unsigned group_count[32][32];  // per-group arrivals (a line per group)
 };
@@ -80,7 +80,7 @@ struct SolveArgs {
     void *pub;                                     // k_cg_local: published rows r, w, s [3][2][n], zeroed
     int salt;                                      // k_cg_local, k_cg_block: stamp of this launch's foreign-read marks
     const int *gate;                               // non-null: the solve is left alone when *gate is 0 (a kernel queued
-                                                   // behind k_cg_block for the systems that one cannot hold)
+                                                   // behind k_cg_block or k_bicg_block for what those cannot hold)
 };
 
 // slot layout of the partial sums (per workgroup and right-hand side)
@@ -292,5 +292,12 @@ BlockKernel cg_block_many(bool f32, int nz, int rpt);
 // batched launch: systems of up to kBlockJobsOne rows on one workgroup, larger ones `rpt` rows per thread on several
 constexpr int kBlockJobsOne = 2048;
 BlockKernel cg_block_jobs(bool f32, int nz, int rpt);
+// k_bicg_block instances: `together` right-hand sides advance at once (nrhs or 1)
+struct BicgBlock {
+    BlockKernel k;
+    int together;
+};
+constexpr int kBicgSums = 9;  // sums of its largest reduction (posted: [4 reductions][2][kBicgSums][workgroup])
+BicgBlock bicg_block(bool f32, int nz, int rpt, int nrhs);
 
 }  // namespace pict

@@ -2082,6 +2082,7 @@ __device__ __forceinline__ void bicg_local(const SolveArgs<float> &a, unsigned b
 
 template <int RPT, int NZ, int NR>
 __global__ __launch_bounds__(kSolveThreads) void k_bicg_local(SolveArgs<float> a) {
+    if (a.gate && *a.gate == 0) return;
     bicg_local<RPT, NZ, NR>(a, blockIdx.x);
 }
 
@@ -2438,6 +2439,7 @@ __device__ __forceinline__ void bicgstab(const SolveArgs<R> &a, unsigned bid) {
 
 template <typename R, int NRHS>
 __global__ __launch_bounds__(kSolveThreads) void k_bicgstab(SolveArgs<R> a) {
+    if (a.gate && *a.gate == 0) return;
     bicgstab<R, NRHS>(a, blockIdx.x);
 }
 
@@ -2625,9 +2627,10 @@ struct Plan {
     bool full;      // k_cg_local reduces the sum and maximum of |r| too
     bool lean;      // k_cg1 without the register row cache
     int cus;        // compute units of the device
-    // k_cg_block in front (null: none); unless it runs on one workgroup, the kernel above is queued behind it for
-    // the systems it cannot hold
+    // k_cg_block or k_bicg_block in front (null: none); unless it runs on one workgroup, the kernel above is queued
+    // behind it for the systems it cannot hold
     BlockKernel block;
+    int block_rhs;  // k_bicg_block: right-hand sides that advance together
     bool block_one;
     int block_nz;
     long long block_nwg;
@@ -2644,6 +2647,13 @@ size_t block_region(long long nwg, long long C, size_t &off) {
     off = (pos / 8 * sizeof(int) + 255) & ~size_t(255);
     return 8 * ((size_t)nwg * 4 + 2 * pos);
 }
+// k_bicg_block's: the same, with `together` right-hand sides and larger reductions
+size_t bicg_tagged_words(long long nwg) { return (size_t)nwg * 8 * kBicgSums; }
+size_t bicg_block_region(long long nwg, long long C, int together, size_t &off) {
+    const size_t pos = (size_t)nwg * C;
+    off = (pos / 8 * sizeof(int) + 255) & ~size_t(255);
+    return 8 * (bicg_tagged_words(nwg) + 2 * pos * together);
+}
 
 // k_cg_block's shape for a system: instance and workgroups, or none (a longer row on average than its registers take,
 // or more rows than fit on the chip).  Measured per iteration, FP32 unless said, before = the kernel of plan_general:
@@ -2658,20 +2668,14 @@ size_t block_region(long long nwg, long long C, size_t &off) {
 //    with two, 2.1 on 50 with four; before: 4.2), a row costs 0.25 us (131 x 67 x 45: 3.1 with four rows, 4.1 with
 //    eight; before: 17.2); 150 x 90 x 60: 25 -> 5.4, 192 x 96 x 96 with fourteen: 40 -> 7.8.
 // PICT_CG_LOCAL_WGS (a workgroup budget of k_cg_local) selects plan_general's kernels.
-template <typename R>
-void plan_block(const pict_csr_desc *A, int cus, Plan &pl) {
-    const long long n = A->n;
-    if ((long long)A->nnz > 7 * n || getenv("PICT_CG_LOCAL_WGS")) return;
-    const bool f32 = sizeof(R) == 4;
-    const int nz = (long long)A->nnz <= 5 * n ? 5 : 7;
-    pl.block_nz = nz;
-    pl.block = cg_block_one(f32, nz, n);
-    pl.block_one = pl.block.kernel != nullptr;
-    pl.block_nwg = 1;
-    if (pl.block_one) return;
+//
+// block_shape: instance and workgroups of a block kernel for n rows, the fewest rows per thread (kernel(rows): its
+// instance, if any) whose grid stays within these limits.
+template <typename F>
+void block_shape(long long n, int nz, int cus, F kernel, Plan &pl) {
     const long long cap = std::min(cus, 256);
     for (int rpt : {1, 2, 4, 8, 14}) {
-        const BlockKernel k = cg_block_many(f32, nz, rpt);
+        const BlockKernel k = kernel(rpt);
         if (!k.kernel) continue;  // (also FP64 5-entry rows, one per thread)
         const long long C = (long long)k.threads * rpt;
         long long nwg = block_wgs(n, C, nz);
@@ -2686,6 +2690,44 @@ void plan_block(const pict_csr_desc *A, int cus, Plan &pl) {
         pl.block_nwg = nwg;
         return;
     }
+}
+
+template <typename R>
+void plan_block(const pict_csr_desc *A, int cus, Plan &pl) {
+    const long long n = A->n;
+    if ((long long)A->nnz > 7 * n || getenv("PICT_CG_LOCAL_WGS")) return;
+    const bool f32 = sizeof(R) == 4;
+    const int nz = (long long)A->nnz <= 5 * n ? 5 : 7;
+    pl.block_nz = nz;
+    pl.block = cg_block_one(f32, nz, n);
+    pl.block_one = pl.block.kernel != nullptr;
+    pl.block_nwg = 1;
+    if (pl.block_one) return;
+    block_shape(n, nz, cus, [&](int rpt) { return cg_block_many(f32, nz, rpt); }, pl);
+}
+
+// k_bicg_block's shape for a system, by the same rule (its trips and rows cost the same, three and two times per
+// iteration).  Measured per solve from zero, all right-hand sides, before = the kernel of plan_general:
+//  - 5-entry rows, two right-hand sides together: 97 x 61 58 -> 37 us (2 iterations), 128 x 100 52 -> 41, 256 x 256 68
+//    -> 52 (65 with four rows per thread), 301 x 203 95 -> 53, 640 x 500 204 -> 109 (134 with eight); one after the
+//    other 1.2-1.4 times as much.  FP64 97 x 61 199 -> 57 (4 iterations), 320 x 256 186 -> 74, 640 x 500 279 -> 149.
+//  - 7-entry rows, three together up to four rows per thread: 24 x 17 x 16 312 -> 91 (6 iterations; 148 one after the
+//    other), 57 x 35 x 30 325 -> 127 (204 with four rows), 131 x 67 x 45 617 -> 295 (361); one after the other 150 x 90
+//    x 60 1072 -> 529, 192 x 96 x 96 1864 -> 738.  FP64 57 x 35 x 30 563 -> 228, 90 x 60 x 40 852 -> 532.
+// Systems of up to kBlockJobsOne rows stay with plan_general: a batch of them runs k_bicg_local_jobs, whose results a
+// single solve of the same system has to match to the bit, and 64 x 64 gains 8 us of 46 only.
+// PICT_BICG_LOCAL=0 and PICT_CG_LOCAL_WGS select plan_general's kernels.
+template <typename R>
+void plan_bicg_block(const pict_csr_desc *A, int nrhs, int cus, Plan &pl) {
+    const long long n = A->n;
+    if (n <= kBlockJobsOne || (long long)A->nnz > 7 * n || !bicg_local_enabled() || getenv("PICT_CG_LOCAL_WGS")) return;
+    const int nz = (long long)A->nnz <= 5 * n ? 5 : 7;
+    pl.block_nz = nz;
+    block_shape(n, nz, cus, [&](int rpt) {
+        const BicgBlock k = bicg_block(sizeof(R) == 4, nz, rpt, nrhs);
+        pl.block_rhs = k.together;
+        return k.k;
+    }, pl);
 }
 
 template <typename R>
@@ -2807,17 +2849,19 @@ pict_status plan_solve(const pict_csr_desc *A, int nrhs, const pict_solve_opts *
     if (pl.kind == Kind::kCG1 && nrhs == 1 && o->residual_reset_steps <= 0 && !o->return_best_result &&
         (o->convergence_criterion == PICT_CONV_NORM2 || o->convergence_criterion == PICT_CONV_NORM2_NORMALIZED))
         plan_block<R>(A, pl.cus, pl);
+    if (pl.kind == Kind::kBiCG &&
+        (o->convergence_criterion == PICT_CONV_NORM2 || o->convergence_criterion == PICT_CONV_NORM2_NORMALIZED))
+        plan_bicg_block<R>(A, nrhs, pl.cus, pl);
     return PICT_OK;
 }
 
 // Workspace of one solve: vectors | FP64 partials | final states | transpose map | control block |
 // k_cg_local's tagged partials and published rows.  The control block and the regions after it
-// are zeroed by one fill kernel before the launch.  k_cg_block's marks, tagged partials and published rows lie in
-// the vectors, which the general kernel only writes after k_cg_block has left the system to it (block_extra: bytes
-// they need beyond the vectors).
+// are zeroed by one fill kernel before the launch.  The marks, tagged partials and published rows of k_cg_block and
+// k_bicg_block lie in the vectors, which the general kernel only writes after they have left the system to it.
 struct Layout {
     size_t vec, off_part, off_st, off_perm, off_ctl, off_zero, words_tagged, words_zero, total;
-    size_t off_block, block_words;  // k_cg_block: tagged partials and published rows
+    size_t off_block, block_words;  // k_cg_block, k_bicg_block: tagged partials and published rows
 };
 
 template <typename R>
@@ -2832,10 +2876,14 @@ Layout layout_of(const pict_csr_desc *A, int nrhs, const pict_solve_opts *o, con
     size_t bytes_vec = sizeof(R) * L.vec * nvec;
     if (pl.block.kernel) {
         const long long C = (long long)pl.block.threads * pl.block.rpt;
-        const size_t bytes = pl.block_one ? 0 : block_region(pl.block_nwg, C, L.off_block);
+        const bool bicg = pl.kind == Kind::kBiCG;
+        const size_t bytes = pl.block_one ? 0
+                             : bicg ? bicg_block_region(pl.block_nwg, C, pl.block_rhs, L.off_block)
+                                    : block_region(pl.block_nwg, C, L.off_block);
         L.block_words = bytes / 8;
-        // (the large instances keep x behind)
-        bytes_vec = std::max<size_t>(bytes_vec, L.off_block + bytes + sizeof(R) * (size_t)(pl.block_nwg * C));
+        // (behind: x in the large instances, k_bicg_block's shadow residuals)
+        const size_t behind = sizeof(R) * (size_t)(pl.block_nwg * C) * (bicg ? pl.block_rhs + 1 : 1);
+        bytes_vec = std::max<size_t>(bytes_vec, L.off_block + bytes + behind);
     }
     L.off_part = al(bytes_vec);
     L.off_st = L.off_part + al(bytes_part);
@@ -2862,7 +2910,7 @@ pict_status enqueue_typed(const pict_csr_desc *A, const void *rhs, void *x, int 
     const void *kernel = pl.kernel;
     const long long nwg = pl.nwg;
     Layout L = layout_of<R>(A, nrhs, o, pl);
-    if (ws_in && ws_bytes < L.total && pl.block.kernel) {  // a caller's workspace without room for k_cg_block
+    if (ws_in && ws_bytes < L.total && pl.block.kernel) {  // a caller's workspace without room for a block kernel
         pl.block.kernel = nullptr;
         L = layout_of<R>(A, nrhs, o, pl);
     }
@@ -2952,7 +3000,7 @@ pict_status enqueue_typed(const pict_csr_desc *A, const void *rhs, void *x, int 
         SolveArgs<R> ba = a;
         ba.p0 = (R *)ws;
         ba.tagged = (unsigned long long *)(ws + L.off_block);
-        ba.pub = ba.tagged + (size_t)pl.block_nwg * 4;
+        ba.pub = ba.tagged + (kind == Kind::kBiCG ? bicg_tagged_words(pl.block_nwg) : (size_t)pl.block_nwg * 4);
         ba.nwg = (unsigned)pl.block_nwg;
         void *bargs[] = {&ba};
         PICT_HIP_TRY(hipLaunchKernel(pl.block.kernel, dim3((unsigned)pl.block_nwg), dim3(pl.block.threads), bargs, 0,
@@ -3593,7 +3641,9 @@ pict_status pict_solver_kernel_name(const pict_csr_desc *A, int32_t nrhs, const 
     st = f32 ? plan_solve<float>(A, nrhs, opts, pl) : plan_solve<double>(A, nrhs, opts, pl);
     if (st) return st;
     const int nr = nrhs < kMaxRhs ? nrhs : kMaxRhs;
-    if (pl.block.kernel)
+    if (pl.block.kernel && pl.kind == Kind::kBiCG)
+        snprintf(buf, (size_t)len, "pict::k_bicg_block<%s, %d, %d, %d>", t, pl.block.rpt, pl.block_nz, pl.block_rhs);
+    else if (pl.block.kernel)
         snprintf(buf, (size_t)len, "pict::k_cg_block<%s, %d, %d, %d, %s>", t, pl.block.threads, pl.block.rpt,
                  pl.block_nz, pl.block_one ? "one" : "several");
     else if (pl.local)
