@@ -582,19 +582,26 @@ __global__ __launch_bounds__(T) void k_cg_block(SolveArgs<R> a) {
 }
 
 // Batched launch (job lists as for k_cg_local_jobs): systems of up to 2048 rows run the one-workgroup instance that
-// they would run alone, larger ones RPT rows per thread.
-template <typename R, int RPT, int NZ, int HPT>
+// they would run alone, larger ones as many rows per thread as the batch's plan gave them.
+template <typename R, int NZ>
 __global__ __launch_bounds__(512) void k_cg_block_jobs(const SolveArgs<R> *__restrict__ args,
                                                        const unsigned *__restrict__ job_off,
                                                        const unsigned *__restrict__ jobs) {
+    constexpr int H2 = NZ <= 5 ? 2 : 4, H4 = NZ <= 5 ? 3 : 6;
+    constexpr bool f32 = sizeof(R) == 4;
     const unsigned j0 = job_off[blockIdx.x], j1 = job_off[blockIdx.x + 1];
     for (unsigned j = j0; j < j1; ++j) {
-        const unsigned job = (unsigned)__builtin_amdgcn_readfirstlane((int)jobs[j]);
-        const SolveArgs<R> a = args[job >> 16];
+        const unsigned job = (unsigned)__builtin_amdgcn_readfirstlane((int)jobs[j]), bid = job & 0xffffu;
+        const SolveArgs<R> a = job_args(args, job);
         if (a.n <= 512) cg_block<R, 512, 1, NZ, 1, false, true>(a, 0);
         else if (a.n <= 1024) cg_block<R, 512, 2, NZ, 1, false, true>(a, 0);
         else if (a.n <= kBlockJobsOne) cg_block<R, 512, 4, NZ, 1, false, true>(a, 0);
-        else cg_block<R, 512, RPT, NZ, HPT, false, false>(a, job & 0xffffu);
+        else if (a.block_rpt == 2) cg_block<R, 512, 2, NZ, H2, false, false>(a, bid);
+        else if (a.block_rpt == 4) {
+            if constexpr (block_jobs_has(f32, NZ, 4)) cg_block<R, 512, 4, NZ, H4, false, false>(a, bid);
+        } else {
+            if constexpr (block_jobs_has(f32, NZ, 8)) cg_block<R, 512, 8, NZ, 4, false, false>(a, bid);
+        }
         __syncthreads();
     }
 }
@@ -645,24 +652,10 @@ BlockKernel cg_block_one(bool f32, int nz, long long n) {
     return f32 ? (nz <= 5 ? one_kernel<float, 5>(n) : one_kernel<float, 7>(n))
                : (nz <= 5 ? one_kernel<double, 5>(n) : one_kernel<double, 7>(n));
 }
-template <typename R, int NZ>
-static BlockKernel jobs_kernel(int rpt) {
-    constexpr int H1 = NZ <= 5 ? 2 : 3, H2 = NZ <= 5 ? 2 : 4, H4 = NZ <= 5 ? 3 : 6;
-    switch (rpt) {
-        case 1: return {(const void *)k_cg_block_jobs<R, 1, NZ, H1>, 512, 1};
-        case 2: return {(const void *)k_cg_block_jobs<R, 2, NZ, H2>, 512, 2};
-        case 4:
-            if constexpr (sizeof(R) == 4 || NZ <= 5) return {(const void *)k_cg_block_jobs<R, 4, NZ, H4>, 512, 4};
-            return {nullptr, 0, 0};
-        case 8:
-            if constexpr (sizeof(R) == 4 && NZ <= 5) return {(const void *)k_cg_block_jobs<R, 8, NZ, 4>, 512, 8};
-            return {nullptr, 0, 0};
-        default: return {nullptr, 0, 0};
-    }
-}
-BlockKernel cg_block_jobs(bool f32, int nz, int rpt) {
-    return f32 ? (nz <= 5 ? jobs_kernel<float, 5>(rpt) : jobs_kernel<float, 7>(rpt))
-               : (nz <= 5 ? jobs_kernel<double, 5>(rpt) : jobs_kernel<double, 7>(rpt));
+BlockKernel cg_block_jobs(bool f32, int nz) {
+    return {f32 ? (nz <= 5 ? (const void *)k_cg_block_jobs<float, 5> : (const void *)k_cg_block_jobs<float, 7>)
+                : (nz <= 5 ? (const void *)k_cg_block_jobs<double, 5> : (const void *)k_cg_block_jobs<double, 7>),
+            512, 0};
 }
 BlockKernel cg_block_many(bool f32, int nz, int rpt) {
     return f32 ? (nz <= 5 ? many_kernel<float, 5>(rpt) : many_kernel<float, 7>(rpt))

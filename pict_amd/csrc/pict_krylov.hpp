@@ -78,10 +78,33 @@ struct SolveArgs {
     unsigned long long *tagged;                    // tagged partials [2][nwg][kSlots], zeroed (k_cg_local packs its
                                                    // NS values per workgroup: [2][nwg][NS])
     void *pub;                                     // k_cg_local: published rows r, w, s [3][2][n], zeroed
+    int block_rpt;                                 // k_cg_block_jobs: rows per thread of a system on several workgroups
     int salt;                                      // k_cg_local, k_cg_block: stamp of this launch's foreign-read marks
     const int *gate;                               // non-null: the solve is left alone when *gate is 0 (a kernel queued
                                                    // behind k_cg_block or k_bicg_block for what those cannot hold)
 };
+
+// The arguments of a system from a table in memory.  A pointer read from memory has no known address space, and an
+// access through it is a flat one, which waits for the LDS counter too; read as a pointer to global memory, it compiles
+// to the same loads as a kernel's own pointer arguments.
+template <typename T>
+__device__ __forceinline__ T *load_global_ptr(T *const *p) {
+    return (T *)*reinterpret_cast<__attribute__((address_space(1))) T *const *>(p);
+}
+template <typename R>
+__device__ __forceinline__ SolveArgs<R> job_args(const SolveArgs<R> *args, unsigned job) {
+    const SolveArgs<R> &in = args[job >> 16];
+    SolveArgs<R> a = in;
+#define PICT_GLOBAL(f) a.f = load_global_ptr(&in.f)
+    PICT_GLOBAL(row), PICT_GLOBAL(col), PICT_GLOBAL(val), PICT_GLOBAL(b), PICT_GLOBAL(x);
+    PICT_GLOBAL(r), PICT_GLOBAL(rhat), PICT_GLOBAL(p0), PICT_GLOBAL(p1), PICT_GLOBAL(v0), PICT_GLOBAL(v1);
+    PICT_GLOBAL(s), PICT_GLOBAL(t), PICT_GLOBAL(best), PICT_GLOBAL(partials), PICT_GLOBAL(ctl), PICT_GLOBAL(st);
+    PICT_GLOBAL(tagged), PICT_GLOBAL(gate);
+#undef PICT_GLOBAL
+    a.pub = load_global_ptr(reinterpret_cast<char *const *>(&in.pub));
+    a.perm = nullptr;  // batched solves are not transposed
+    return a;
+}
 
 // slot layout of the partial sums (per workgroup and right-hand side)
 enum { S_RR = 0, S_ASUM = 1, S_AMAX = 2, S_D0 = 3, S_D1 = 4, S_BMAX = 5 };
@@ -289,9 +312,13 @@ struct BlockKernel {
 };
 BlockKernel cg_block_one(bool f32, int nz, long long n);
 BlockKernel cg_block_many(bool f32, int nz, int rpt);
-// batched launch: systems of up to kBlockJobsOne rows on one workgroup, larger ones `rpt` rows per thread on several
+// batched launch: systems of up to kBlockJobsOne rows on one workgroup, larger ones SolveArgs::block_rpt rows per thread
+// on several (those for which block_jobs_has holds)
 constexpr int kBlockJobsOne = 2048;
-BlockKernel cg_block_jobs(bool f32, int nz, int rpt);
+BlockKernel cg_block_jobs(bool f32, int nz);
+constexpr bool block_jobs_has(bool f32, int nz, int rpt) {
+    return rpt == 2 || (rpt == 4 && (f32 || nz <= 5)) || (rpt == 8 && f32 && nz <= 5);
+}
 // k_bicg_block instances: `together` right-hand sides advance at once (nrhs or 1)
 struct BicgBlock {
     BlockKernel k;

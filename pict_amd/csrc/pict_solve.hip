@@ -1679,7 +1679,7 @@ __global__ __launch_bounds__(kSolveThreads) void k_cg_local_jobs(const SolveArgs
     const unsigned j0 = job_off[blockIdx.x], j1 = job_off[blockIdx.x + 1];
     for (unsigned j = j0; j < j1; ++j) {
         const unsigned job = jobs[j];
-        const SolveArgs<R> a = args[job >> 16];
+        const SolveArgs<R> a = job_args(args, job);
         if (a.gate && *a.gate == 0) continue;  // solved by k_cg_block_jobs
         cg_local<R, RPT, NZ, FULL>(a, job & 0xffffu);
         __syncthreads();
@@ -2094,7 +2094,7 @@ __global__ __launch_bounds__(kSolveThreads) void k_bicg_local_jobs(const SolveAr
     const unsigned j0 = job_off[blockIdx.x], j1 = job_off[blockIdx.x + 1];
     for (unsigned j = j0; j < j1; ++j) {
         const unsigned job = jobs[j];
-        const SolveArgs<float> a = args[job >> 16];
+        const SolveArgs<float> a = job_args(args, job);
         bicg_local<RPT, NZ, NR>(a, job & 0xffffu);
         __syncthreads();
     }
@@ -2451,7 +2451,7 @@ __global__ __launch_bounds__(kSolveThreads) void k_bicgstab_jobs(const SolveArgs
     const unsigned j0 = job_off[blockIdx.x], j1 = job_off[blockIdx.x + 1];
     for (unsigned j = j0; j < j1; ++j) {
         const unsigned job = jobs[j];
-        const SolveArgs<R> a = args[job >> 16];
+        const SolveArgs<R> a = job_args(args, job);
         bicgstab<R, NRHS>(a, job & 0xffffu);
         __syncthreads();
     }
@@ -3114,7 +3114,7 @@ struct BatchSolve {
     const void *block = nullptr;
     unsigned block_grid = 0;
     bool coop = true;  // the general kernel is a cooperative launch
-    std::vector<int> block_nwg;
+    std::vector<int> block_nwg, block_rpt;  // (rows per thread; 0: one workgroup)
     size_t off_bargs = 0, off_bjoboff = 0, off_bjobs = 0;
     std::vector<char> bargs_host;
     std::vector<unsigned> bjob_off, bjobs;
@@ -3244,6 +3244,59 @@ std::vector<double> default_cost(const BatchSolve &b) {
     return c;
 }
 
+// Workgroups and rows per thread (at most `most`) of every system in k_cg_block_jobs, `cap` workgroups resident; false
+// if a system does not fit.  A solve waits for the longest of its workgroups' lists, so the plan that promises the
+// shortest one is taken: the same rows per thread for all, or the most rows for all and then step by step half as many
+// for the system that takes longest.  64 lid cavities of 32 x 32 to 248 x 248 (720 iterations): 2.3 ms with four rows for
+// all, in two rounds, 2.5 ms with eight in one, 1.7 ms with this plan.
+bool plan_block_jobs(BatchSolve &b, bool f32, int most, long long cap) {
+    // us per iteration (256 x 256 on 32 workgroups and more), one workgroup: by rows; iterations like the square root
+    auto cost = [&](int s, int rpt) {
+        const double t = rpt == 0 ? 0.6 + 0.7 * b.n[s] / kBlockJobsOne : rpt == 2 ? 1.8 : rpt == 4 ? 2.1 : 2.9;
+        return t * std::sqrt((double)b.n[s]);
+    };
+    auto wgs = [&](int s, int rpt) { return rpt == 0 ? 1LL : block_wgs(b.n[s], 512LL * rpt, b.nz); };
+    const long long sys_cap = std::min<long long>(cap, 256);
+    double best = -1.0;
+    std::vector<int> rpts(b.count), nwg(b.count);
+    std::vector<double> costs(b.count);
+    std::vector<unsigned> off, jobs;
+    auto consider = [&]() -> bool {  // keeps the plan in rpts if it is the best so far
+        long long sum = 0;
+        for (int s = 0; s < b.count; ++s) {
+            const long long w = wgs(s, rpts[s]);
+            if (w > sys_cap) return false;
+            nwg[s] = (int)w;
+            costs[s] = cost(s, rpts[s]);
+            sum += w;
+        }
+        const double m = schedule(b.count, nwg, (unsigned)std::min(sum, cap), costs, off, jobs);
+        if (best >= 0.0 && m >= best) return false;
+        best = m;
+        b.block_nwg = nwg;
+        b.block_rpt = rpts;
+        return true;
+    };
+    int top = 0;
+    // (one row per thread takes no less time than two)
+    for (int rpt = 2; rpt <= std::max(most, 2); rpt *= 2) {
+        if (!block_jobs_has(f32, b.nz, rpt)) continue;
+        for (int s = 0; s < b.count; ++s) rpts[s] = b.n[s] <= kBlockJobsOne ? 0 : rpt;
+        consider();
+        top = rpt;
+    }
+    // (a step that does not help by itself, such as one of two equal systems, may with the next)
+    for (int step = 0, worse = 0; top > 0 && step < 64 && worse < 4; ++step) {
+        int last = 0;
+        for (int s = 1; s < b.count; ++s)
+            if (cost(s, rpts[s]) > cost(last, rpts[last])) last = s;
+        if (rpts[last] < 4) break;
+        rpts[last] /= 2;
+        worse = consider() ? 0 : worse + 1;
+    }
+    return best >= 0.0;
+}
+
 template <typename R>
 void fill_args(BatchSolve &b, int s, const pict_csr_desc &A, const void *rhs, void *x, const pict_solve_opts *o,
                const std::vector<size_t> &off_vec, const std::vector<size_t> &off_part,
@@ -3284,6 +3337,7 @@ void fill_args(BatchSolve &b, int s, const pict_csr_desc &A, const void *rhs, vo
     if (b.block) {
         SolveArgs<R> ba = a;  // the marks lie in the vectors (p0)
         ba.nwg = (unsigned)b.block_nwg[s];
+        ba.block_rpt = b.block_rpt[s];
         ba.tagged = reinterpret_cast<unsigned long long *>(b.arena + off_blk[s]);
         ba.pub = ba.tagged + (size_t)ba.nwg * 4;
         memcpy(b.bargs_host.data() + (size_t)s * sizeof ba, &ba, sizeof ba);
@@ -3362,22 +3416,18 @@ pict_status batch_create_typed(const pict_csr_desc *A, const void *const *rhs, v
         sum += w;
     }
     b->grid = (unsigned)std::min(sum, cap);
-    // k_cg_block_jobs in front, for the same rows per thread, when every system's workgroups can be resident
+    // k_cg_block_jobs in front, when every system's workgroups can be resident
     if (b->local && !o->return_best_result && !getenv("PICT_CG_LOCAL_WGS")) {
-        const BlockKernel k = cg_block_jobs(sizeof(R) == 4, b->nz, b->rpt);
+        const BlockKernel k = cg_block_jobs(sizeof(R) == 4, b->nz);
         int bocc = 0, bcus = 0;
-        if (k.kernel && (st = occupancy(k.kernel, bocc, bcus, k.threads))) return st;
-        const long long C = (long long)k.threads * k.rpt, bcap = std::min<long long>((long long)bocc * bcus, 256);
-        bool fits = k.kernel && bocc > 0;
-        long long bsum = 0;
-        b->block_nwg.assign(count, 1);
-        for (int s = 0; s < count && fits; ++s) {
-            if (A[s].n > kBlockJobsOne) b->block_nwg[s] = (int)std::min<long long>(block_wgs(A[s].n, C, b->nz), 65535);
-            fits = b->block_nwg[s] <= bcap && (long long)A[s].nnz <= 7LL * A[s].n;
-            bsum += b->block_nwg[s];
-        }
-        if (fits) {
+        if ((st = occupancy(k.kernel, bocc, bcus, k.threads))) return st;
+        bool fits = bocc > 0;
+        for (int s = 0; s < count && fits; ++s) fits = (long long)A[s].nnz <= 7LL * A[s].n;
+        const int most = cfg.rows_per_thread > 0 ? cfg.rows_per_thread : 8;
+        if (fits && plan_block_jobs(*b, sizeof(R) == 4, most, (long long)bocc * bcus)) {
             b->block = k.kernel;
+            long long bsum = 0;
+            for (int w : b->block_nwg) bsum += w;
             b->block_grid = (unsigned)std::min<long long>(bsum, (long long)bocc * bcus);
             b->bargs_host.assign(sizeof(SolveArgs<R>) * count, 0);
             // the general kernel then usually has nothing to do: one workgroup per compute unit, an ordinary launch
@@ -3428,7 +3478,7 @@ pict_status batch_create_typed(const pict_csr_desc *A, const void *const *rhs, v
         if (b->block) {
             size_t marks = 0;
             off_blk[s] = off;
-            if (b->n[s] > kBlockJobsOne) off += al(block_region(b->block_nwg[s], 512LL * b->rpt, marks));
+            if (b->n[s] > kBlockJobsOne) off += al(block_region(b->block_nwg[s], 512LL * b->block_rpt[s], marks));
         }
     }
     b->zero_words = (off - b->off_zero) / sizeof(unsigned long long);
@@ -3545,8 +3595,7 @@ void batch_solve_describe(const BatchSolve *b, BatchSolveInfo *out) {
     out->makespan = b->makespan;
     const bool f32 = b->dtype == PICT_DTYPE_F32;
     if (b->block)
-        snprintf(out->kernel, sizeof out->kernel, "pict::k_cg_block_jobs<%s, %d, %d>", f32 ? "float" : "double", b->rpt,
-                 b->nz);
+        snprintf(out->kernel, sizeof out->kernel, "pict::k_cg_block_jobs<%s, %d>", f32 ? "float" : "double", b->nz);
     else if (b->local)
         snprintf(out->kernel, sizeof out->kernel, "pict::k_cg_local_jobs<%s, %d, %d, false>", f32 ? "float" : "double",
                  b->rpt, b->nz);
