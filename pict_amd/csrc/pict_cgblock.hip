@@ -253,7 +253,10 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
     // wave 0, with `mid` run by waves 1.. once the workgroup's partials are out.  False in wave 0 (else
     // ignored) when a wait ran out.
     auto reduce = [&](unsigned gen, bool max1, double &t0, double &t1, auto mid) -> bool {
-        if constexpr (!ONE && !kTagged) ops_done();  // published rows before the partials
+        // before the partials: the halo marks, which their owners read once after the first totals, and FP64 rows (FP32
+        // rows carry their iteration)
+        if constexpr (!ONE)
+            if (!kTagged || gen == 0u) ops_done();
         const int par = (int)(gen & 1u);
         if (max1) {
             const double w0 = wave_reduce_dpp<false>(acc0), w1 = wave_reduce_dpp<true>(acc1);
