@@ -360,7 +360,7 @@ typedef struct pict_solve_info {     /* LinearSolverResultInfo, bicgstab_solver.
     int32_t used_iterations;
     int32_t converged;
     int32_t is_finite_residual;
-    int32_t reserved;
+    int32_t reserved;                /* 1: a kernel with the state on chip solved it (pict_solve_refined: sweeps) */
 } pict_solve_info;
 
 /* SolveLinear (PISOtorch.cpp:559-563; PISO_multiblock_cuda_kernel.cu:7021-7103,

@@ -101,11 +101,12 @@ class Int4:
 class LinearSolverResultInfo:
     """bicgstab_solver.h:20-25."""
 
-    def __init__(self, finalResidual, usedIterations, converged, isFiniteResidual):
+    def __init__(self, finalResidual, usedIterations, converged, isFiniteResidual, onChip=False):
         self.finalResidual = float(finalResidual)
         self.usedIterations = int(usedIterations)
         self.converged = bool(converged)
         self.isFiniteResidual = bool(isFiniteResidual)
+        self.onChip = bool(onChip)  # solved by a kernel that holds the system's state on chip (diagnostics)
 
     def __str__(self):
         return ("LinearSolverResultInfo(finalResidual=%g, usedIterations=%d, converged=%d, isFiniteResidual=%d)"
@@ -2244,7 +2245,7 @@ def _solve(A, RHS, x, opts):
     _abi.check(lib.pict_solve_linear(ctypes.byref(desc), ctypes.c_void_p(RHS.data_ptr()),
                                      ctypes.c_void_p(x.data_ptr()), nb, ctypes.byref(opts), infos,
                                      _stream(RHS.device)), "SolveLinear")
-    res = [LinearSolverResultInfo(i.final_residual, i.used_iterations, i.converged, i.is_finite_residual)
+    res = [LinearSolverResultInfo(i.final_residual, i.used_iterations, i.converged, i.is_finite_residual, i.reserved)
            for i in infos]
     if solve_log is not None:
         solve_log.append(("BiCG" if opts.use_bicg else "CG", n, A.getSize(), nb, RHS.element_size(), res,

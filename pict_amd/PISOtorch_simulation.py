@@ -845,7 +845,7 @@ class Simulation:
         domain = self.domain
         D, K = domain.getSpatialDims(), o.corrector_steps
         res = [PISOtorch.LinearSolverResultInfo(i.final_residual, i.used_iterations, i.converged,
-                                                i.is_finite_residual) for i in infos]
+                                                i.is_finite_residual, i.reserved) for i in infos]
         adv, prs = res[:D], res[D:]
         akind = "BiCG" if self.advection_use_BiCG else "CG"
         pkind = "BiCG" if self.pressure_use_BiCG else "CG"

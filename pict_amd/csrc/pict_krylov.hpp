@@ -58,7 +58,8 @@ struct RhsState {
     int active, converged, finite, used;
     int best_it, rising, save_best, restore_best;
     double final_res;
-    double pad;
+    int on_chip;  // k_cg_block or k_bicg_block solved it (filled in with the caller's copy)
+    int pad;
 };
 
 template <typename R>

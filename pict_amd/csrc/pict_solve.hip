@@ -2173,11 +2173,16 @@ __global__ __launch_bounds__(256) void k_refine_update(double *x, const R *d, do
     for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) x[i] += scale * (double)d[i];
 }
 
-// a solve's final states and barrier error flag to the caller's slots (one launch after the solver kernel)
-__global__ void k_solve_out(const RhsState *st, int nrhs, const int *err, RhsState *st_out, int *err_out) {
+// a solve's final states and barrier error flag to the caller's slots (one launch after the solver kernel); block: a
+// block kernel was queued, which solved the system unless it left it (zero_all)
+__global__ void k_solve_out(const RhsState *st, int nrhs, const Ctl *ctl, bool block, RhsState *st_out, int *err_out) {
     const int k = threadIdx.x;
-    if (k < nrhs) st_out[k] = st[k];
-    if (k == 0) *err_out = *err;
+    if (k < nrhs) {
+        RhsState s = st[k];
+        s.on_chip = block && ctl->zero_all == 0;
+        st_out[k] = s;
+    }
+    if (k == 0) *err_out = ctl->err;
 }
 
 // zero n (and m) 64-bit words (control block and tagged regions, before a solver kernel's launch)
@@ -3014,8 +3019,8 @@ pict_status enqueue_typed(const pict_csr_desc *A, const void *rhs, void *x, int 
     else
         PICT_HIP_TRY(hipLaunchCooperativeKernel(kernel, dim3((unsigned)nwg), dim3(kSolveThreads), args, 0, stream));
     if (ev1) PICT_HIP_TRY(hipEventRecord(ev1, stream));
-    hipLaunchKernelGGL(k_solve_out, dim3(1), dim3(64), 0, stream, (const RhsState *)a.st, nrhs,
-                       (const int *)&a.ctl->err, state_out, err_out);
+    hipLaunchKernelGGL(k_solve_out, dim3(1), dim3(64), 0, stream, (const RhsState *)a.st, nrhs, (const Ctl *)a.ctl,
+                       pl.block.kernel != nullptr, state_out, err_out);
     PICT_HIP_TRY(hipGetLastError());
     return PICT_OK;
 }
@@ -3083,7 +3088,7 @@ void solve_state_to_info(const void *states, int nrhs, pict_solve_info *out) {
         out[k].used_iterations = hs[k].used;
         out[k].converged = hs[k].converged;
         out[k].is_finite_residual = hs[k].finite;
-        out[k].reserved = 0;
+        out[k].reserved = hs[k].on_chip;
     }
 }
 
@@ -3163,14 +3168,17 @@ const void *bicgstab_jobs_kernel(int nrhs) {
     }
 }
 
-// OR of the systems' barrier error flags
+// OR of the systems' barrier error flags; each system's final states learn which kernel solved it
 template <typename R>
 __global__ __launch_bounds__(256) void k_batch_err(const SolveArgs<R> *args, int count, int *out) {
     __shared__ int any;
     if (threadIdx.x == 0) any = 0;
     __syncthreads();
-    for (int s = threadIdx.x; s < count; s += blockDim.x)
+    for (int s = threadIdx.x; s < count; s += blockDim.x) {
         if (__hip_atomic_load(&args[s].ctl->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(&any, 1);
+        const int on_chip = args[s].gate && *args[s].gate == 0;
+        for (int k = 0; k < args[s].nrhs; ++k) args[s].st[k].on_chip = on_chip;
+    }
     __syncthreads();
     if (threadIdx.x == 0) *out = any;
 }

@@ -42,7 +42,8 @@ def test_mixed_rows_match_single_steps(name, rows, dtype):
     doms, sims = _sims(BATCHES[name], dtype)
     batch = SimulationBatch(sims, config=dict(pressure_rows_per_thread=rows))
     for _ in range(2):
-        batch.step()
+        infos = batch.step()
+    assert (infos["reserved"][:, 2:] == 1).all()  # the pressure solves ran on chip, not only by plan
     info = batch.describe()
     assert "k_cg_block_jobs" in info["pressure_kernel"], info
     tol = 1e-10 if dtype == torch.float64 else 1e-6

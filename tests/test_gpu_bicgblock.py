@@ -52,7 +52,7 @@ def check_residual(m, x, b, k, tol):
     assert r <= bound, (k, r, bound)
 
 
-def check(m, nr, dtype, name_part, monkeypatch):
+def check(m, nr, dtype, name_part, monkeypatch, on_chip=True):
     A, n = to_pict(m, dtype), m.shape[0]
     b = rhs(n, nr, 3, dtype)
     b[:n] *= 1e-2  # the right-hand sides end at different iterations
@@ -61,11 +61,13 @@ def check(m, nr, dtype, name_part, monkeypatch):
     assert name_part in name, name
     tol = 1e-12 if dtype == F64 else 1e-6
     x, infos = solve(A, b, tol)
+    assert all(i.onChip == on_chip for i in infos)  # which kernel solved it, not only which one was planned
     x2, _ = solve(A, b, tol)
     assert torch.equal(x, x2)
     monkeypatch.setenv("PICT_CG_LOCAL_WGS", "64")
     assert "k_bicg_block" not in P.solver_kernel_name(A, nr, opts(1e-6))
     _, ref = solve(A, b, tol)
+    assert not any(i.onChip for i in ref)
     monkeypatch.delenv("PICT_CG_LOCAL_WGS")
     for k in range(nr):
         assert infos[k].converged and infos[k].isFiniteResidual and infos[k].finalResidual < tol
@@ -84,7 +86,8 @@ def test_2d(shape, rpt, nr, monkeypatch):
 @pytest.mark.parametrize("shape,rpt", [((683, 4), 2), ((97, 61), 2), ((363, 362), 4)])
 @pytest.mark.parametrize("nr", [1, 2, 3])
 def test_2d_fp64(shape, rpt, nr, monkeypatch):
-    check(skewed(shape, periodic_laplacian), nr, F64, "<double, %d, 5, %d>" % (rpt, 2 if nr == 2 else 1), monkeypatch)
+    check(skewed(shape, periodic_laplacian), nr, F64, "<double, %d, 5, %d>" % (rpt, 2 if nr == 2 else 1), monkeypatch,
+          on_chip=2 * shape[0] <= 896)
 
 
 # 7-entry rows: blocks of lines that do not divide the grid; three together up to four rows per thread
@@ -106,13 +109,13 @@ def test_3d_fp64(shape, rpt, nr, monkeypatch):
 @pytest.mark.parametrize("dtype", [F64, F32])
 def test_left_to_the_general_kernel(dtype, monkeypatch):
     """Lines too long for the halo, columns all over the system, rows longer than the registers."""
-    check(skewed((3000, 4)), 2, dtype, "k_bicg_block", monkeypatch)
-    check(irregular(20000, 3), 2, dtype, "", monkeypatch)
+    check(skewed((3000, 4)), 2, dtype, "k_bicg_block", monkeypatch, on_chip=False)
+    check(irregular(20000, 3), 2, dtype, "", monkeypatch, on_chip=False)
     m = walls((120, 100), 0.05).tolil()
     m[0, ::1500] = -0.01  # one row of 10 entries and its mirror
     m[::1500, 0] = -0.01
     m[0, 0] = 5.0
-    check(m.tocsr(), 2, dtype, "k_bicg_block", monkeypatch)
+    check(m.tocsr(), 2, dtype, "k_bicg_block", monkeypatch, on_chip=False)
 
 
 @pytest.mark.parametrize("shape,nr", [((96, 64), 2), ((96, 64), 3), ((33, 20, 21), 3)])
@@ -126,6 +129,7 @@ def test_transposed(shape, nr, dtype):
     assert "k_bicg_block" in P.solver_kernel_name(A, nr, opts(1e-6))
     xt, it = solve(A, b, 1e-6, transpose=True)
     xe, ie = solve(At, b, 1e-6)
+    assert all(i.onChip for i in it + ie)
     assert [i.usedIterations for i in it] == [i.usedIterations for i in ie] and torch.equal(xt, xe)
 
 
@@ -141,7 +145,7 @@ def test_limits_zero_and_not_finite(shape, nr):
     # the iteration limit: the residual after it is reported
     x, infos = solve(A, b, 1e-30, maxit=3)
     for k, info in enumerate(infos):
-        assert info.usedIterations == 2 and not info.converged and info.isFiniteResidual
+        assert info.onChip and info.usedIterations == 2 and not info.converged and info.isFiniteResidual
         r = b[k * n:(k + 1) * n].double().cpu().numpy() - m @ x[k * n:(k + 1) * n].double().cpu().numpy()
         r = np.linalg.norm(r) / np.sqrt(n)
         assert abs(r - info.finalResidual) <= 1e-3 * r + 1e-7

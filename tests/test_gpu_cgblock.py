@@ -33,7 +33,7 @@ def walls(shape, shift):
     return m
 
 
-def check(m, dtype, name_part, monkeypatch, seed=3):
+def check(m, dtype, name_part, monkeypatch, seed=3, on_chip=True):
     A = to_pict(m, dtype)
     n = m.shape[0]
     b = rhs(n, seed, dtype)
@@ -43,10 +43,12 @@ def check(m, dtype, name_part, monkeypatch, seed=3):
     tol = 1e-12 if dtype == torch.float64 else 1e-6
     x, info = solve(A, b, tol)
     assert info.converged and info.isFiniteResidual
+    assert info.onChip == on_chip  # which kernel solved it, not only which one was planned
     x2, info2 = solve(A, b, tol)
     assert info2.usedIterations == info.usedIterations and torch.equal(x, x2)
     monkeypatch.setenv("PICT_CG_LOCAL_WGS", "64")
     xr, ir = solve(A, b, tol)
+    assert not ir.onChip
     monkeypatch.delenv("PICT_CG_LOCAL_WGS")
     assert abs(info.usedIterations - ir.usedIterations) <= 2 + 0.03 * ir.usedIterations
     xn = x.double().cpu().numpy()
@@ -79,12 +81,13 @@ def test_one_workgroup_1024_threads(shape, monkeypatch):
 def test_several_workgroups_2d(shape, rpt, build, monkeypatch):
     if build is periodic_laplacian and min(shape) < 3:
         shape = (1366, 3)
-    check(build(shape, 0.05), torch.float32, "512, %d, 5, several" % rpt, monkeypatch)
+    # (two whole lines are more than the 896 halo rows from 449 cells on)
+    check(build(shape, 0.05), torch.float32, "512, %d, 5, several" % rpt, monkeypatch, on_chip=2 * shape[0] <= 896 or shape[1] == 1)
 
 
 @pytest.mark.parametrize("shape", [(683, 4), (97, 61), (181, 182)])
 def test_several_workgroups_2d_fp64(shape, monkeypatch):
-    check(walls(shape, 0.05), torch.float64, "several", monkeypatch)
+    check(walls(shape, 0.05), torch.float64, "several", monkeypatch, on_chip=2 * shape[0] <= 896)
 
 
 # 3-D: blocks of lines that do not divide the grid, planes larger and smaller than a workgroup
@@ -103,14 +106,14 @@ def test_several_workgroups_3d_fp64(shape, monkeypatch):
 def test_left_to_the_general_kernel(dtype, monkeypatch):
     """Lines too long for the halo, columns all over the system, and rows longer than the registers: the general
     kernel solves them; on one workgroup long rows are read from memory."""
-    check(walls((3000, 4), 0.05), dtype, "several", monkeypatch)
-    check(irregular(20000, 3), dtype, "", monkeypatch)
+    check(walls((3000, 4), 0.05), dtype, "several", monkeypatch, on_chip=False)
+    check(irregular(20000, 3), dtype, "", monkeypatch, on_chip=False)
     n = 12000
     m = walls((120, 100), 0.05).tolil()
     m[0, ::1500] = -0.01  # one row of 10 entries and its mirror
     m[::1500, 0] = -0.01
     m[0, 0] = 5.0
-    check(m.tocsr(), dtype, "several", monkeypatch)
+    check(m.tocsr(), dtype, "several", monkeypatch, on_chip=False)
     m = walls((30, 30), 0.05).tolil()
     m[0, ::90] = -0.01
     m[::90, 0] = -0.01
@@ -130,6 +133,7 @@ def test_transposed(shape):
         assert "k_cg_block" in kernel_name(A)
         xt, it = solve(A, b, 1e-6, transpose=True, maxit=200)
         xe, ie = solve(At, b, 1e-6, maxit=200)
+        assert it.onChip and ie.onChip
         assert it.usedIterations == ie.usedIterations and torch.equal(xt, xe)
 
 
@@ -145,7 +149,7 @@ def test_limits_zero_and_not_finite(shape):
     assert torch.equal(x, x0) and info.usedIterations == -1 and not info.converged
     # the iteration limit: the residual after it is reported
     x, info = solve(A, b, 1e-30, maxit=7)
-    assert info.usedIterations == 6 and not info.converged and info.isFiniteResidual
+    assert info.onChip and info.usedIterations == 6 and not info.converged and info.isFiniteResidual
     r = np.linalg.norm(b.double().cpu().numpy() - m @ x.double().cpu().numpy()) / np.sqrt(n)
     assert abs(r - info.finalResidual) <= 1e-4 * r
     # the zero right-hand-side shortcut
