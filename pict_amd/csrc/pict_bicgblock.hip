@@ -25,7 +25,8 @@
 // 128 workgroups, 2 for 256) and, with 14 rows per thread, two products of 3.5 us.  Figures stand at plan_bicg_block
 // (pict_solve.hip).
 //
-// A system that the kernel cannot hold is left to the general kernel, as in k_cg_block.
+// A system that the kernel cannot hold, or whose grid does not become resident, is left to the general kernel, as in
+// k_cg_block.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -59,11 +60,11 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
     __shared__ int scan[kBW];
     __shared__ unsigned key[2];
     __shared__ BlockMap m;
-    __shared__ int s_over, s_err;
+    __shared__ int s_over, s_err, s_late, s_go;
     const unsigned bid = blockIdx.x;
     const int t = (int)threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     int herr = 0;
-    if (t == 0) s_over = s_err = 0;
+    if (t == 0) s_over = s_err = s_late = 0;
     block_map<T, C, NZ>(a.row, a.col, a.n, (int)a.nwg, m, key);
     __syncthreads();
     if (bid >= (unsigned)m.nwg) return;
@@ -131,7 +132,7 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
     };
 
     // Reduce-barrier: the totals of acc[0..S) over all workgroups in tot, sum S - 1 a maximum if MAXLAST.  `mid` is run
-    // by waves 1.. once their partials are out.  False in every thread when a wait ran out.
+    // by waves 1.. once their partials are out.  False in every thread when a wait ran out, or the grid declined.
     auto reduce = [&](int red, unsigned gen, auto maxlast, auto &acc, auto mid) -> bool {
         constexpr int S = (int)(sizeof(acc) / sizeof(acc[0]));
         constexpr bool MAXLAST = decltype(maxlast)::value;
@@ -167,47 +168,72 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
             }
         }
         if (wave > 0) mid();
+        // the totals: false after `limit` polls, or once the grid has declined (admit, may be null)
+        auto poll = [&](unsigned limit, const int *admit) {
+            bool ok = true;
 #pragma unroll
-        for (int s0 = 0; s0 < S; s0 += kBW) {
-            const int s = s0 + wave;
-            if (s < S) {
-                const bool mx = MAXLAST && s == S - 1;
-                const u64 *set = post + (size_t)s * nwg;
-                double v;
-                unsigned spins = 0;
-                bool ok = true;
-                for (;;) {
-                    u64 u[4];
-                    bool ready = true;
-                    v = 0.0;
+            for (int s0 = 0; s0 < S; s0 += kBW) {
+                const int s = s0 + wave;
+                if (s < S) {
+                    const bool mx = MAXLAST && s == S - 1;
+                    const u64 *set = post + (size_t)s * nwg;
+                    double v;
+                    unsigned spins = 0;
+                    for (;;) {
+                        u64 u[4];
+                        bool ready = true;
+                        v = 0.0;
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        if (64u * j >= nwg) continue;
-                        const unsigned w = (unsigned)lane + 64u * j;
-                        u[j] = ld_coh(set + (w < nwg ? w : 0u));
-                    }
+                        for (int j = 0; j < 4; ++j) {
+                            if (64u * j >= nwg) continue;
+                            const unsigned w = (unsigned)lane + 64u * j;
+                            u[j] = ld_coh(set + (w < nwg ? w : 0u));
+                        }
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        if ((unsigned)lane + 64u * j >= nwg) continue;
-                        ready = ready & partial_ready(u[j], gen);
-                        const double q = partial_value(u[j]);
-                        v = mx ? fmax(v, q) : v + q;
+                        for (int j = 0; j < 4; ++j) {
+                            if ((unsigned)lane + 64u * j >= nwg) continue;
+                            ready = ready & partial_ready(u[j], gen);
+                            const double q = partial_value(u[j]);
+                            v = mx ? fmax(v, q) : v + q;
+                        }
+                        if (__all(ready)) break;
+                        if (++spins > limit) {
+                            ok = false;
+                            break;
+                        }
+                        if (admit) {
+                            if (ld_coh(admit) == kAdmitDecline) {
+                                ok = false;
+                                break;
+                            }
+                            wait_long(spins);
+                        }
                     }
-                    if (__all(ready)) break;
-                    if (++spins > kSpinLimit) {
-                        ok = false;
-                        break;
-                    }
-                }
-                const double g = mx ? wave_reduce_dpp<true>(v) : wave_reduce_dpp<false>(v);
-                if (lane == 0) {
-                    tot[s] = g;
-                    if (!ok) {
-                        st_coh(&a.ctl->err, 1);
-                        s_err = 1;
-                    }
+                    const double g = mx ? wave_reduce_dpp<true>(v) : wave_reduce_dpp<false>(v);
+                    if (lane == 0) tot[s] = g;
                 }
             }
+            return ok;
+        };
+        bool ok;
+        if (red == kRedFirst && gen == 0u) {
+            ok = a.admit > 0 && poll(a.admit, &a.ctl->admit);
+            if (!ok && lane == 0) s_late = 1;
+            __syncthreads();
+            if (wave == 0) {
+                const bool go = block_admit(a.ctl, bid, !s_late);
+                if (lane == 0) s_go = go;
+            }
+            __syncthreads();
+            if (!s_go) return false;
+            // admitted by workgroup 0 while this wait ran out: everything is posted
+            if (!ok) ok = poll(kSpinLimit, nullptr);
+        } else {
+            ok = poll(kSpinLimit, nullptr);
+        }
+        if (!ok && lane == 0) {
+            st_coh(&a.ctl->err, 1);
+            s_err = 1;
         }
         __syncthreads();
         return s_err == 0;

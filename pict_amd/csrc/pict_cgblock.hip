@@ -28,8 +28,9 @@
 // TB/s); figures for other sizes stand at plan_block (pict_solve.hip).
 //
 // A system of several workgroups that this kernel cannot hold (a longer row, too many halo rows, no block
-// partition) is left alone: the kernel sets ctl->zero_all ("not solved") before it writes x, and the general
-// kernel queued behind it runs; otherwise that kernel returns at once.
+// partition) is left alone, and so is any system while the grid does not become resident as a whole (block_admit): the
+// kernel sets ctl->zero_all ("not solved") before it writes x, and the general kernel queued behind it runs; otherwise
+// that kernel returns at once.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -40,9 +41,10 @@ namespace pict {
 
 // Totals of one generation over the workgroups' tagged pairs (lane l: workgroups l, l + 64, ... in that
 // order, then across the lanes): the same bits in every workgroup.  At most 256 workgroups; B of a lane's in flight.
+// False after `limit` polls, or once the grid has declined (admit, may be null).
 template <int B>
-__device__ __forceinline__ bool block_poll(const u64 *part, unsigned nwg, unsigned gen, bool max1, double &t0,
-                                           double &t1) {
+__device__ __forceinline__ bool block_poll(const u64 *part, unsigned nwg, unsigned gen, bool max1, unsigned limit,
+                                           const int *admit, double &t0, double &t1) {
     const unsigned lane = threadIdx.x & 63;
     const u64 *set = part + (size_t)(gen & 1u) * nwg * 2;
     double v0, v1;
@@ -72,7 +74,11 @@ __device__ __forceinline__ bool block_poll(const u64 *part, unsigned nwg, unsign
             }
         }
         if (__all(ready)) break;
-        if (++spins > kSpinLimit) return false;
+        if (++spins > limit) return false;
+        if (admit) {
+            if (ld_coh(admit) == kAdmitDecline) return false;
+            wait_long(spins);
+        }
     }
     if (max1) {
         t0 = wave_reduce_dpp<false>(v0);
@@ -138,7 +144,7 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
     __shared__ int scan[kBW];
     __shared__ unsigned key[2];
     __shared__ BlockMap m;
-    __shared__ int s_over, s_err;
+    __shared__ int s_over, s_err, s_declined;
     struct Step {
         double alpha, beta;
         int active;
@@ -147,7 +153,7 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
     // the wave number as a scalar: a wave takes its branch alone, without the other branch's waits
     const int t = (int)threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     int herr = 0;
-    if (t == 0) s_over = s_err = 0;
+    if (t == 0) s_over = s_err = s_declined = 0;
     if constexpr (ONE) {
         if (t == 0) m = BlockMap{a.n, 1};
         __syncthreads();
@@ -249,14 +255,15 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
         g1 = lane_d(v, kBW);
     };
 
-    // Reduce-barrier: the totals of acc0 (sum) and acc1 (sum, or maximum).  ONE: in every thread; else in
+    // Reduce-barrier: the totals of acc0 (sum) and acc1 (sum; of the first reduction maximum).  ONE: in every thread; else in
     // wave 0, with `mid` run by waves 1.. once the workgroup's partials are out.  False in wave 0 (else
     // ignored) when a wait ran out.
-    auto reduce = [&](unsigned gen, bool max1, double &t0, double &t1, auto mid) -> bool {
+    auto reduce = [&](auto first_one, unsigned gen, double &t0, double &t1, auto mid) -> bool {
+        constexpr bool max1 = decltype(first_one)::value;
         // before the partials: the halo marks, which their owners read once after the first totals, and FP64 rows (FP32
         // rows carry their iteration)
         if constexpr (!ONE)
-            if (!kTagged || gen == 0u) ops_done();
+            if (!kTagged || max1) ops_done();
         const int par = (int)(gen & 1u);
         if (max1) {
             const double w0 = wave_reduce_dpp<false>(acc0), w1 = wave_reduce_dpp<true>(acc1);
@@ -276,7 +283,18 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
             double g0, g1;
             wg_totals(par, max1, g0, g1);
             if (lane < 2) st_coh(a.tagged + ((size_t)par * nwg + bid) * 2 + lane, tag_partial(lane ? g1 : g0, gen));
-            ok = block_poll<BIG ? 2 : 4>(a.tagged, nwg, gen, max1, t0, t1);
+            auto poll = [&](unsigned limit, const int *admit) {
+                return block_poll<BIG ? 2 : 4>(a.tagged, nwg, gen, max1, limit, admit, t0, t1);
+            };
+            if (max1 && a.admit != kAdmitAlways) {
+                ok = a.admit > 0 && poll(a.admit, &a.ctl->admit);
+                const bool go = block_admit(a.ctl, bid, ok);
+                if (lane == 0) s_declined = !go;
+                // admitted by workgroup 0 while this wait ran out: everything is posted
+                if (go && !ok) ok = poll(kSpinLimit, nullptr);
+            } else {
+                ok = poll(kSpinLimit, nullptr);
+            }
         } else {
             mid();
         }
@@ -295,15 +313,15 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
     unsigned pubm = 0;  // bit q: the wave publishes its rows q (the same in all its lanes)
     // ---- first totals: (r0, r0), max|b| (infinite: some workgroup cannot hold its rows) ----
     {
-        const bool ok = reduce(0u, true, t0, t1, [] {});
+        const bool ok = reduce(std::true_type{}, 0u, t0, t1, [] {});
         if constexpr (ONE) {
             if (t == 0) bc = Step{t0, t1, 1};
         } else if (t == 0) {
-            if (!ok) fail();
+            if (!ok && !s_declined) fail();
             bc = Step{t0, t1, 1};
         }
         __syncthreads();
-        if (s_err) return;
+        if (s_err || s_declined) return;
         t0 = bc.alpha;
         t1 = bc.beta;
         if constexpr (!ONE) {
@@ -440,7 +458,7 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
     product(0, 2u);
     {
         double g0, g1 = 0.0;
-        const bool ok = reduce(1u, false, g0, g1, [&] { prefetch_halo(0, 2u); });
+        const bool ok = reduce(std::false_type{}, 1u, g0, g1, [&] { prefetch_halo(0, 2u); });
         auto start = [&](CgRun &r) {
             r.rho = g0;
             r.den = g1;
@@ -510,7 +528,7 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
         __syncthreads();
         product((it + 1) & 1, (unsigned)it + 3u);
         double gam = 0.0, delta = 0.0;
-        const bool ok = reduce((unsigned)it + 2u, false, gam, delta, [&] {
+        const bool ok = reduce(std::false_type{}, (unsigned)it + 2u, gam, delta, [&] {
             if constexpr (BIG) {
                 constexpr int XB = 4;  // rows of x in flight per thread
                 static_assert(!BIG || C % (XB * kBF) == 0, "whole batches");

@@ -21,8 +21,9 @@ struct Ctl {
     unsigned gen;                // barrier generation
     unsigned pad1[31];
     int err;                     // a wait exceeded its spin limit
-    int zero_all;                // k_cg: every right-hand side is zero; k_cg_block, k_bicg_block: the system does not fit
-    unsigned pad2[30];
+    int zero_all;                // k_cg: every right-hand side is zero; k_cg_block, k_bicg_block: not solved there
+    int admit;                   // k_cg_block, k_bicg_block: kAdmit*
+    unsigned pad2[29];
     unsigned group_count[32][32];  // per-group arrivals (a line per group)
 };
 // Resident workgroups (256 threads) per compute unit that a persistent solver grid is sized for.  Grids of seven
@@ -81,6 +82,9 @@ struct SolveArgs {
     void *pub;                                     // k_cg_local: published rows r, w, s [3][2][n], zeroed
     int block_rpt;                                 // k_cg_block_jobs: rows per thread of a system on several workgroups
     int salt;                                      // k_cg_local, k_cg_block: stamp of this launch's foreign-read marks
+    unsigned admit;                                // k_cg_block, k_bicg_block: polls of the first totals before the grid
+                                                   // declines (block_admit; 0: it does); kAdmitAlways: resident by
+                                                   // its launch
     const int *gate;                               // non-null: the solve is left alone when *gate is 0 (a kernel queued
                                                    // behind k_cg_block or k_bicg_block for what those cannot hold)
 };
@@ -105,6 +109,41 @@ __device__ __forceinline__ SolveArgs<R> job_args(const SolveArgs<R> *args, unsig
     a.pub = load_global_ptr(reinterpret_cast<char *const *>(&in.pub));
     a.perm = nullptr;  // batched solves are not transposed
     return a;
+}
+
+// Admission of a block kernel's grid.  Its workgroups wait for each other, so all of them have to be resident, and an
+// ordinary launch does not promise that: two such grids on concurrent streams (or in two processes) can each hold a part
+// of the compute units.  Nothing is written before the first totals, whose wait therefore decides: workgroup 0 admits the
+// grid once it has seen the partial sums of all workgroups, any workgroup whose wait runs out declines it, whichever
+// comes first holds for all (one word), and a grid that declines leaves the system to the general kernel queued behind
+// it.  A grid that is admitted is resident as a whole and always ends, so waiting for one is safe too.
+// The limit, kAdmitPolls, is some 8 ms of polling: longer than most solves that hold the compute units, short against
+// the general kernel's solve of a system this size.  Deciding costs one trip through memory per solve (1 us).
+enum { kAdmitOpen = 0, kAdmitGo = 1, kAdmitDecline = 2 };
+constexpr unsigned kAdmitPolls = 1u << 12;
+constexpr unsigned kAdmitAlways = ~0u;
+// between two polls of a wait that has been long
+__device__ __forceinline__ void wait_long(unsigned spins) {
+    if (spins > 64) __builtin_amdgcn_s_sleep(32);
+}
+// The grid's decision, by one wave (the same in all its lanes); all_posted: this wave has seen every partial sum.
+__device__ __forceinline__ bool block_admit(Ctl *ctl, unsigned bid, bool all_posted) {
+    int d = kAdmitOpen;
+    if ((threadIdx.x & 63) == 0) {
+        if (all_posted && bid != 0) {  // workgroup 0 is resident and decides
+            for (unsigned spins = 0; spins < kSpinLimit && (d = ld_coh(&ctl->admit)) == kAdmitOpen; ++spins)
+                wait_long(spins);
+        }
+        if (d == kAdmitOpen) {
+            const int mine = all_posted && bid == 0 ? kAdmitGo : kAdmitDecline;
+            if (__hip_atomic_compare_exchange_strong(&ctl->admit, &d, mine, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT)) {
+                d = mine;
+                if (mine == kAdmitDecline) st_coh(&ctl->zero_all, 1);
+            }
+        }
+    }
+    return __builtin_amdgcn_readfirstlane(d) == kAdmitGo;
 }
 
 // slot layout of the partial sums (per workgroup and right-hand side)

@@ -2598,14 +2598,30 @@ const void *bicg_local_kernel(int rpt, int nz, int nrhs) {
 // 16.8 M cells*steps/s).  Residency: on an idle device the dispatcher places all of a grid of at most one
 // workgroup per CU at once.  Work of other queues that holds CUs delays the workgroups that find no room, and
 // they start when it releases them; kernels that never wait on other grids (every stage kernel, torch's kernels)
-// always do, so the grid becomes fully resident and its barriers complete.  Two persistent grids that wait on their own barriers and
-// together exceed what the CUs hold (two such solves on concurrent streams, or in two processes sharing the GPU)
-// can each be partly resident; the spin limit then ends the waiting solve with PICT_ERR_DEVICE_SYNC instead of a
-// hang.  The library's own solves are queued on one stream per call, so this only arises from concurrent callers.
+// always do, so the grid becomes fully resident and its barriers complete.  Two persistent grids that wait on their own
+// barriers and together exceed what the CUs hold (solves on concurrent streams, or in two processes sharing the GPU)
+// can each be partly resident.  The block kernels, whose workgroups may fill a CU each (512 threads, up to 158 KB of
+// LDS), find that out before they write anything and leave the solve to the kernel queued behind them (block_admit).
+// For the other kernels, workgroups of 256 threads of which a CU holds several, the spin limit then ends the waiting
+// solve with PICT_ERR_DEVICE_SYNC instead of a hang.  The library's own solves are queued on one stream per call, so
+// this only arises from concurrent callers.
 // PICT_SOLVER_PLAIN_LAUNCH=0 keeps the cooperative launch, whose residency the runtime checks.
 static bool plain_launch_enabled() {
     const char *e = getenv("PICT_SOLVER_PLAIN_LAUNCH");
     return !e || atoi(e) != 0;
+}
+static pict_status launch_solver(const void *kernel, long long nwg, int threads, void **args, int cus,
+                                 hipStream_t stream) {
+    if (plain_launch_enabled() && nwg <= cus)
+        PICT_HIP_TRY(hipLaunchKernel(kernel, dim3((unsigned)nwg), dim3((unsigned)threads), args, 0, stream));
+    else
+        PICT_HIP_TRY(hipLaunchCooperativeKernel(kernel, dim3((unsigned)nwg), dim3((unsigned)threads), args, 0, stream));
+    return PICT_OK;
+}
+// polls before the grid of a block kernel declines (PICT_SOLVER_ADMIT_POLLS; 0: always)
+static unsigned admit_polls() {
+    const char *e = getenv("PICT_SOLVER_ADMIT_POLLS");
+    return e ? (unsigned)std::min(std::max(atoi(e), 0), 1 << 20) : kAdmitPolls;
 }
 // PICT_BICG_LOCAL=0 keeps BiCGStab on the streaming kernel
 static bool bicg_local_enabled() {
@@ -2676,8 +2692,9 @@ size_t bicg_block_region(long long nwg, long long C, int together, size_t &off) 
 //
 // block_shape: instance and workgroups of a block kernel for n rows, the fewest rows per thread (kernel(rows): its
 // instance, if any) whose grid stays within these limits.
+// An instance counts only if it can be resident (one workgroup per compute unit is all that the limits ask for).
 template <typename F>
-void block_shape(long long n, int nz, int cus, F kernel, Plan &pl) {
+pict_status block_shape(long long n, int nz, int cus, F kernel, Plan &pl) {
     const long long cap = std::min(cus, 256);
     for (int rpt : {1, 2, 4, 8, 14}) {
         const BlockKernel k = kernel(rpt);
@@ -2691,24 +2708,29 @@ void block_shape(long long n, int nz, int cus, F kernel, Plan &pl) {
             nwg = std::min(nwg, cap);
         }
         if (nwg > limit) continue;
+        int occ = 0, c = 0;
+        pict_status st = occupancy(k.kernel, occ, c, k.threads);
+        if (st) return st;
+        if (occ < 1) continue;
         pl.block = k;
         pl.block_nwg = nwg;
-        return;
+        return PICT_OK;
     }
+    return PICT_OK;
 }
 
 template <typename R>
-void plan_block(const pict_csr_desc *A, int cus, Plan &pl) {
+pict_status plan_block(const pict_csr_desc *A, int cus, Plan &pl) {
     const long long n = A->n;
-    if ((long long)A->nnz > 7 * n || getenv("PICT_CG_LOCAL_WGS")) return;
+    if ((long long)A->nnz > 7 * n || getenv("PICT_CG_LOCAL_WGS")) return PICT_OK;
     const bool f32 = sizeof(R) == 4;
     const int nz = (long long)A->nnz <= 5 * n ? 5 : 7;
     pl.block_nz = nz;
     pl.block = cg_block_one(f32, nz, n);
     pl.block_one = pl.block.kernel != nullptr;
     pl.block_nwg = 1;
-    if (pl.block_one) return;
-    block_shape(n, nz, cus, [&](int rpt) { return cg_block_many(f32, nz, rpt); }, pl);
+    if (pl.block_one) return PICT_OK;
+    return block_shape(n, nz, cus, [&](int rpt) { return cg_block_many(f32, nz, rpt); }, pl);
 }
 
 // k_bicg_block's shape for a system, by the same rule (its trips and rows cost the same, three and two times per
@@ -2723,12 +2745,13 @@ void plan_block(const pict_csr_desc *A, int cus, Plan &pl) {
 // single solve of the same system has to match to the bit, and 64 x 64 gains 8 us of 46 only.
 // PICT_BICG_LOCAL=0 and PICT_CG_LOCAL_WGS select plan_general's kernels.
 template <typename R>
-void plan_bicg_block(const pict_csr_desc *A, int nrhs, int cus, Plan &pl) {
+pict_status plan_bicg_block(const pict_csr_desc *A, int nrhs, int cus, Plan &pl) {
     const long long n = A->n;
-    if (n <= kBlockJobsOne || (long long)A->nnz > 7 * n || !bicg_local_enabled() || getenv("PICT_CG_LOCAL_WGS")) return;
+    if (n <= kBlockJobsOne || (long long)A->nnz > 7 * n || !bicg_local_enabled() || getenv("PICT_CG_LOCAL_WGS"))
+        return PICT_OK;
     const int nz = (long long)A->nnz <= 5 * n ? 5 : 7;
     pl.block_nz = nz;
-    block_shape(n, nz, cus, [&](int rpt) {
+    return block_shape(n, nz, cus, [&](int rpt) {
         const BicgBlock k = bicg_block(sizeof(R) == 4, nz, rpt, nrhs);
         pl.block_rhs = k.together;
         return k.k;
@@ -2853,10 +2876,10 @@ pict_status plan_solve(const pict_csr_desc *A, int nrhs, const pict_solve_opts *
     if (st) return st;
     if (pl.kind == Kind::kCG1 && nrhs == 1 && o->residual_reset_steps <= 0 && !o->return_best_result &&
         (o->convergence_criterion == PICT_CONV_NORM2 || o->convergence_criterion == PICT_CONV_NORM2_NORMALIZED))
-        plan_block<R>(A, pl.cus, pl);
+        return plan_block<R>(A, pl.cus, pl);
     if (pl.kind == Kind::kBiCG &&
         (o->convergence_criterion == PICT_CONV_NORM2 || o->convergence_criterion == PICT_CONV_NORM2_NORMALIZED))
-        plan_bicg_block<R>(A, nrhs, pl.cus, pl);
+        return plan_bicg_block<R>(A, nrhs, pl.cus, pl);
     return PICT_OK;
 }
 
@@ -3007,17 +3030,13 @@ pict_status enqueue_typed(const pict_csr_desc *A, const void *rhs, void *x, int 
         ba.tagged = (unsigned long long *)(ws + L.off_block);
         ba.pub = ba.tagged + (kind == Kind::kBiCG ? bicg_tagged_words(pl.block_nwg) : (size_t)pl.block_nwg * 4);
         ba.nwg = (unsigned)pl.block_nwg;
+        ba.admit = admit_polls();
         void *bargs[] = {&ba};
-        PICT_HIP_TRY(hipLaunchKernel(pl.block.kernel, dim3((unsigned)pl.block_nwg), dim3(pl.block.threads), bargs, 0,
-                                     stream));
+        if ((st = launch_solver(pl.block.kernel, pl.block_nwg, pl.block.threads, bargs, pl.cus, stream))) return st;
         a.gate = &a.ctl->zero_all;
     }
-    if (pl.block.kernel && pl.block_one)
-        ;
-    else if (plain_launch_enabled() && nwg <= pl.cus)
-        PICT_HIP_TRY(hipLaunchKernel(kernel, dim3((unsigned)nwg), dim3(kSolveThreads), args, 0, stream));
-    else
-        PICT_HIP_TRY(hipLaunchCooperativeKernel(kernel, dim3((unsigned)nwg), dim3(kSolveThreads), args, 0, stream));
+    if (!pl.block.kernel || !pl.block_one)
+        if ((st = launch_solver(kernel, nwg, kSolveThreads, args, pl.cus, stream))) return st;
     if (ev1) PICT_HIP_TRY(hipEventRecord(ev1, stream));
     hipLaunchKernelGGL(k_solve_out, dim3(1), dim3(64), 0, stream, (const RhsState *)a.st, nrhs, (const Ctl *)a.ctl,
                        pl.block.kernel != nullptr, state_out, err_out);
@@ -3346,6 +3365,7 @@ void fill_args(BatchSolve &b, int s, const pict_csr_desc &A, const void *rhs, vo
         SolveArgs<R> ba = a;  // the marks lie in the vectors (p0)
         ba.nwg = (unsigned)b.block_nwg[s];
         ba.block_rpt = b.block_rpt[s];
+        ba.admit = kAdmitAlways;  // (a cooperative launch)
         ba.tagged = reinterpret_cast<unsigned long long *>(b.arena + off_blk[s]);
         ba.pub = ba.tagged + (size_t)ba.nwg * 4;
         memcpy(b.bargs_host.data() + (size_t)s * sizeof ba, &ba, sizeof ba);
