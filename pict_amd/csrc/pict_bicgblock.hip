@@ -63,7 +63,6 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
     __shared__ int s_over, s_err, s_late, s_go;
     const unsigned bid = blockIdx.x;
     const int t = (int)threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    int herr = 0;
     if (t == 0) s_over = s_err = s_late = 0;
     block_map<T, C, NZ>(a.row, a.col, a.n, (int)a.nwg, m, key);
     __syncthreads();
@@ -227,9 +226,9 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
             __syncthreads();
             if (!s_go) return false;
             // admitted by workgroup 0 while this wait ran out: everything is posted
-            if (!ok) ok = poll(kSpinLimit, nullptr);
+            if (!ok) ok = poll(a.spin, nullptr);
         } else {
-            ok = poll(kSpinLimit, nullptr);
+            ok = poll(a.spin, nullptr);
         }
         if (!ok && lane == 0) {
             st_coh(&a.ctl->err, 1);
@@ -253,7 +252,8 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
 #pragma unroll
         for (int j = 0; j < HPT; ++j) hpos[j] = halo_pos(j);
     }
-    // FP32: load until every halo word of the vector carries `tag` (bounded); FP64: one load
+    // FP32: load until every halo word of the vector carries `tag` (bounded: the workgroup then ends with the reduction
+    // under way, so that no other wait is begun); FP64: one load
     auto fetch_halo = [&](int vec, int k, unsigned tag, auto store) {
         constexpr int HB = BIG ? HPT / 2 : HPT;  // BIG: half of the words at a time (registers)
         static_assert(HPT % HB == 0, "whole batches");
@@ -274,8 +274,11 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
                     stale |= mine ? 0u : 1u;
                 }
                 if (!__any(any_halo && stale)) break;
-                if (++spins > kSpinLimit) {
-                    herr = 1;
+                if (++spins > a.spin) {
+                    if (lane == 0) {
+                        st_coh(&a.ctl->err, 1);
+                        s_err = 1;
+                    }
                     break;
                 }
             }
@@ -628,7 +631,6 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
             }
         }
     }
-    if (herr) st_coh(&a.ctl->err, 1);
 }
 
 // Instances: NR = nrhs right-hand sides together, or one after the other (BicgBlock::together).

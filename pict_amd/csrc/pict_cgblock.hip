@@ -152,7 +152,6 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
     __shared__ Step bc;
     // the wave number as a scalar: a wave takes its branch alone, without the other branch's waits
     const int t = (int)threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    int herr = 0;
     if (t == 0) s_over = s_err = s_declined = 0;
     if constexpr (ONE) {
         if (t == 0) m = BlockMap{a.n, 1};
@@ -291,9 +290,9 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
                 const bool go = block_admit(a.ctl, bid, ok);
                 if (lane == 0) s_declined = !go;
                 // admitted by workgroup 0 while this wait ran out: everything is posted
-                if (go && !ok) ok = poll(kSpinLimit, nullptr);
+                if (go && !ok) ok = poll(a.spin, nullptr);
             } else {
-                ok = poll(kSpinLimit, nullptr);
+                ok = poll(a.spin, nullptr);
             }
         } else {
             mid();
@@ -363,7 +362,8 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
 #pragma unroll
         for (int k = 0; k < HPT; ++k) hpos[k] = halo_pos(k);
     }
-    // FP32: load until every halo word carries `tag` (bounded); FP64: one load
+    // FP32: load until every halo word carries `tag` (bounded: the workgroup then ends at its next barrier, so that no
+    // other wait is begun); FP64: one load
     auto fetch_halo = [&](int par, unsigned tag) {
         if constexpr (!ONE) {
             // BIG: half of the words at a time (registers)
@@ -387,8 +387,8 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
                         stale |= mine ? 0u : 1u;
                     }
                     if (!__any(any_halo && stale)) break;
-                    if (++spins > kSpinLimit) {
-                        herr = 1;
+                    if (++spins > a.spin) {
+                        if (lane == 0) fail();
                         break;
                     }
                 }
@@ -564,7 +564,6 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
             cs = bc;
         }
     }
-    if (herr) st_coh(&a.ctl->err, 1);
     if constexpr (BIG) {
         for (int k = h0; k < C && wave > 0; k += kBF) {
             const int i = block_row<C>(m, bid, (unsigned)k);

@@ -85,6 +85,7 @@ struct SolveArgs {
     unsigned admit;                                // k_cg_block, k_bicg_block: polls of the first totals before the grid
                                                    // declines (block_admit; 0: it does); kAdmitAlways: resident by
                                                    // its launch
+    unsigned spin;                                 // k_cg_block, k_bicg_block: polls of every later wait
     const int *gate;                               // non-null: the solve is left alone when *gate is 0 (a kernel queued
                                                    // behind k_cg_block or k_bicg_block for what those cannot hold)
 };

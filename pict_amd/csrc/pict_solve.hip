@@ -2623,6 +2623,11 @@ static unsigned admit_polls() {
     const char *e = getenv("PICT_SOLVER_ADMIT_POLLS");
     return e ? (unsigned)std::min(std::max(atoi(e), 0), 1 << 20) : kAdmitPolls;
 }
+// polls of a block kernel's other waits (PICT_SOLVER_SPIN_LIMIT)
+static unsigned spin_limit() {
+    const char *e = getenv("PICT_SOLVER_SPIN_LIMIT");
+    return e ? (unsigned)std::min(std::max(atoi(e), 0), (int)kSpinLimit) : kSpinLimit;
+}
 // PICT_BICG_LOCAL=0 keeps BiCGStab on the streaming kernel
 static bool bicg_local_enabled() {
     const char *e = getenv("PICT_BICG_LOCAL");
@@ -3031,6 +3036,7 @@ pict_status enqueue_typed(const pict_csr_desc *A, const void *rhs, void *x, int 
         ba.pub = ba.tagged + (kind == Kind::kBiCG ? bicg_tagged_words(pl.block_nwg) : (size_t)pl.block_nwg * 4);
         ba.nwg = (unsigned)pl.block_nwg;
         ba.admit = admit_polls();
+        ba.spin = spin_limit();
         void *bargs[] = {&ba};
         if ((st = launch_solver(pl.block.kernel, pl.block_nwg, pl.block.threads, bargs, pl.cus, stream))) return st;
         a.gate = &a.ctl->zero_all;
@@ -3366,6 +3372,7 @@ void fill_args(BatchSolve &b, int s, const pict_csr_desc &A, const void *rhs, vo
         ba.nwg = (unsigned)b.block_nwg[s];
         ba.block_rpt = b.block_rpt[s];
         ba.admit = kAdmitAlways;  // (a cooperative launch)
+        ba.spin = kSpinLimit;
         ba.tagged = reinterpret_cast<unsigned long long *>(b.arena + off_blk[s]);
         ba.pub = ba.tagged + (size_t)ba.nwg * 4;
         memcpy(b.bargs_host.data() + (size_t)s * sizeof ba, &ba, sizeof ba);

@@ -123,3 +123,18 @@ def test_launch_kinds(shape, dtype, bicg, general, monkeypatch):
         assert on_chip == (not general)
         out.append(x)
     assert torch.equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("shape,dtype,bicg", CASES)
+def test_a_wait_that_runs_out_ends_the_solve(shape, dtype, bicg, monkeypatch):
+    """With no polls allowed after admission the first wait that is not over at once ends its workgroup and then the
+    others: an error, no second wait, and the next solve is not affected."""
+    print("case", shape, dtype, bicg, flush=True)
+    A, b = system(shape, dtype, bicg)
+    x, _ = both(A, b, bicg, monkeypatch)
+    monkeypatch.setenv("PICT_SOLVER_SPIN_LIMIT", "0")
+    with pytest.raises(Exception, match="spin limit"):
+        solve(A, b, bicg)
+    monkeypatch.delenv("PICT_SOLVER_SPIN_LIMIT")
+    z, on_chip = solve(A, b, bicg)
+    assert on_chip and torch.equal(z, x)
