@@ -35,8 +35,13 @@
 
 namespace pict {
 
-// posted partial sums: [reduction of an iteration (kRed*)][parity][sum][workgroup]
+// reductions: a group's first, then three per iteration
 enum { kRedFirst, kRedA, kRedB, kRedC };
+// set of posted partial sums of a reduction's generation (kBicgSets)
+__device__ __forceinline__ unsigned bicg_set(int red, unsigned gen) {
+    return red == kRedFirst ? gen : (unsigned)(kMaxRhs + 2 * (red - kRedA)) + (gen & 1u);
+}
+static_assert(kBicgSets == kMaxRhs + 6, "sets of posted sums");
 
 // a wave-uniform value, held in scalar registers
 __device__ __forceinline__ double uniform_d(double v) { return lane_d(v, 0); }
@@ -151,7 +156,8 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
             if (lane == 0) wsum[S - 1][wave] = w;
         }
         __syncthreads();
-        u64 *post = a.tagged + (size_t)(red * 2 + (int)(gen & 1u)) * kSums * nwg;
+        const unsigned row = post_stride(nwg);
+        u64 *post = a.tagged + (size_t)(bicg_set(red, gen) * kSums * row);
 #pragma unroll
         for (int s0 = 0; s0 < S; s0 += kBW) {
             const int s = s0 + wave;
@@ -163,19 +169,20 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
                 v = op(v, dpp_d<0xB1>(v));   // quad_perm [1,0,3,2]
                 v = op(v, dpp_d<0x4E>(v));   // quad_perm [2,3,0,1]
                 v = op(v, dpp_d<0x141>(v));  // row_half_mirror
-                if (lane == 0) st_coh(post + (size_t)s * nwg + bid, tag_partial(v, gen));
+                if (lane == 0) st_coh(post + (size_t)s * row + bid, post_word(v));
             }
         }
         if (wave > 0) mid();
+        ops_done();  // before polling (kCgSets)
         // the totals: false after `limit` polls, or once the grid has declined (admit, may be null)
         auto poll = [&](unsigned limit, const int *admit) {
-            bool ok = true;
+            bool ok = !admit || limit > 0u;
 #pragma unroll
             for (int s0 = 0; s0 < S; s0 += kBW) {
                 const int s = s0 + wave;
                 if (s < S) {
                     const bool mx = MAXLAST && s == S - 1;
-                    const u64 *set = post + (size_t)s * nwg;
+                    const u64 *set = post + (size_t)s * row;
                     double v;
                     unsigned spins = 0;
                     for (;;) {
@@ -191,8 +198,8 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
 #pragma unroll
                         for (int j = 0; j < 4; ++j) {
                             if ((unsigned)lane + 64u * j >= nwg) continue;
-                            ready = ready & partial_ready(u[j], gen);
-                            const double q = partial_value(u[j]);
+                            ready = ready & (u[j] != 0);
+                            const double q = post_value(u[j]);
                             v = mx ? fmax(v, q) : v + q;
                         }
                         if (__all(ready)) break;
@@ -215,8 +222,9 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
             return ok;
         };
         bool ok;
-        if (red == kRedFirst && gen == 0u) {
-            ok = a.admit > 0 && poll(a.admit, &a.ctl->admit);
+        for (bool admit = red == kRedFirst && gen == 0u;; admit = false) {
+            ok = poll(admit ? a.admit : a.spin, admit ? &a.ctl->admit : nullptr);
+            if (!admit) break;
             if (!ok && lane == 0) s_late = 1;
             __syncthreads();
             if (wave == 0) {
@@ -225,14 +233,20 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
             }
             __syncthreads();
             if (!s_go) return false;
-            // admitted by workgroup 0 while this wait ran out: everything is posted
-            if (!ok) ok = poll(a.spin, nullptr);
-        } else {
-            ok = poll(a.spin, nullptr);
+            if (ok) break;  // else workgroup 0 admitted the grid while this wait ran out: everything is posted
         }
         if (!ok && lane == 0) {
             st_coh(&a.ctl->err, 1);
             s_err = 1;
+        }
+        // clear the words of the next reduction of this kind (all workgroups have read them: they have posted this one);
+        // complete before this workgroup polls the next reduction of any kind, so before the post that lets others read
+        // them
+        if (red != kRedFirst) {
+            u64 *next = a.tagged + (size_t)(bicg_set(red, gen + 1u) * kSums * row);
+#pragma unroll
+            for (int s0 = 0; s0 < S; s0 += kBW)
+                if (lane == 0 && s0 + wave < S) st_coh(next + (size_t)(s0 + wave) * row + bid, (u64)0);
         }
         __syncthreads();
         return s_err == 0;

@@ -39,14 +39,14 @@
 
 namespace pict {
 
-// Totals of one generation over the workgroups' tagged pairs (lane l: workgroups l, l + 64, ... in that
+// Totals of one generation over the workgroups' posted pairs (lane l: workgroups l, l + 64, ... in that
 // order, then across the lanes): the same bits in every workgroup.  At most 256 workgroups; B of a lane's in flight.
 // False after `limit` polls, or once the grid has declined (admit, may be null).
 template <int B>
 __device__ __forceinline__ bool block_poll(const u64 *part, unsigned nwg, unsigned gen, bool max1, unsigned limit,
                                            const int *admit, double &t0, double &t1) {
     const unsigned lane = threadIdx.x & 63;
-    const u64 *set = part + (size_t)(gen & 1u) * nwg * 2;
+    const u64 *set = part + (size_t)((gen & (kCgSets - 1)) * post_stride(2 * nwg));
     double v0, v1;
     unsigned spins = 0;
     for (;;) {
@@ -67,9 +67,9 @@ __device__ __forceinline__ bool block_poll(const u64 *part, unsigned nwg, unsign
 #pragma unroll
             for (int j = 0; j < B; ++j) {
                 if (lane + 64u * (b + j) >= nwg) continue;
-                ready = ready && partial_ready(u[j][0], gen) && partial_ready(u[j][1], gen);
-                v0 += partial_value(u[j][0]);
-                const double q = partial_value(u[j][1]);
+                ready = ready & (u[j][0] != 0) & (u[j][1] != 0);
+                v0 += post_value(u[j][0]);
+                const double q = post_value(u[j][1]);
                 v1 = max1 ? fmax(v1, q) : v1 + q;
             }
         }
@@ -93,9 +93,11 @@ __device__ __forceinline__ bool block_poll(const u64 *part, unsigned nwg, unsign
 
 // The scalar step of cg_run_update (pict_krylov.hpp) for the norm-2 criteria without best-result bookkeeping; the
 // criterion's square root is taken only near the tolerance and at the end (final_res: block_run_end).
-template <typename R>
+// FP64 systems take quotients as rounded as a division's (DIV); of FP32 systems the coefficients are rounded to FP32
+// afterwards, and on one workgroup every wave forms them (rcp64, as in k_cg_local: 1.27 instead of 1.34 us, 75 x 54).
+template <bool DIV, typename R>
 __device__ __forceinline__ void block_run_update(const SolveArgs<R> &a, CgRun &st, double gam, double delta, int it) {
-    const double beta_n = gam * st.inv_rho;
+    const double beta_n = DIV ? div64(gam, st.rho, st.inv_rho) : gam * st.inv_rho;
     const double den_n = fma(-beta_n * beta_n, st.den, delta);
     st.used = it;
     const double near = gam * (a.crit_scale * a.crit_scale);
@@ -109,7 +111,7 @@ __device__ __forceinline__ void block_run_update(const SolveArgs<R> &a, CgRun &s
             return;
         }
     }
-    st.alpha = gam * rcp64(den_n);
+    st.alpha = DIV ? div64(gam, den_n, rcp64(den_n)) : gam * rcp64(den_n);
     st.beta = beta_n;
     st.den = den_n;
     st.rho = gam;
@@ -281,7 +283,12 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
         } else if (wave == 0) {
             double g0, g1;
             wg_totals(par, max1, g0, g1);
-            if (lane < 2) st_coh(a.tagged + ((size_t)par * nwg + bid) * 2 + lane, tag_partial(lane ? g1 : g0, gen));
+            auto slot = [&](unsigned g) {
+                return a.tagged + (size_t)((g & (kCgSets - 1)) * post_stride(2 * nwg) + 2 * bid + (unsigned)lane);
+            };
+            if (lane < 2) st_coh(slot(gen), post_word(lane ? g1 : g0));
+            if (lane < 2) st_coh(slot(gen + 2u), (u64)0);
+            ops_done();
             auto poll = [&](unsigned limit, const int *admit) {
                 return block_poll<BIG ? 2 : 4>(a.tagged, nwg, gen, max1, limit, admit, t0, t1);
             };
@@ -543,7 +550,7 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
             prefetch_halo((it + 1) & 1, (unsigned)it + 3u);
         });
         if constexpr (ONE) {
-            block_run_update(a, run, gam, delta, it);
+            block_run_update<false>(a, run, gam, delta, it);
             cs = Step{run.alpha, run.beta, run.active};
         } else {
             if (wave == 0) {
@@ -551,11 +558,11 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
                     if (t == 0) fail();
                 } else if constexpr (kRunLds) {
                     if (t == 0) {
-                        block_run_update(a, srun, gam, delta, it);
+                        block_run_update<sizeof(R) == 8>(a, srun, gam, delta, it);
                         bc = Step{srun.alpha, srun.beta, srun.active};
                     }
                 } else {
-                    block_run_update(a, run, gam, delta, it);
+                    block_run_update<sizeof(R) == 8>(a, run, gam, delta, it);
                     if (t == 0) bc = Step{run.alpha, run.beta, run.active};
                 }
             }

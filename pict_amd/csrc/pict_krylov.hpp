@@ -202,6 +202,24 @@ __device__ __forceinline__ u64 tag_partial(double v, unsigned gen) {
 __device__ __forceinline__ bool partial_ready(u64 u, unsigned gen) { return (unsigned)(u & 3u) == ((gen + 1u) & 3u); }
 __device__ __forceinline__ double partial_value(u64 u) { return __longlong_as_double((long long)(u & ~3ull)); }
 
+// Partial sums as k_cg_block and k_bicg_block post them: whole, a word that is not posted yet is 0 (+0 travels as -0,
+// which adds the same).  The sets of words rotate, and a set is used again only after its owner has cleared its words.
+// CG: with its post of generation g a workgroup clears its words of set g + 2 (every workgroup has posted g - 1, so all
+// have read g - 2, the same set), and it waits for both stores before it polls, so before its post of g + 1, without
+// which nobody reads set g + 2.  BiCGStab's other reductions lie between two of a kind, so that two sets do; the words
+// are cleared behind the totals.
+// That wait, for all stores of a wave before it begins to poll, is also the faster way: polls that begin while stores
+// are under way slow them (CG per iteration with it and without: 256 x 256 1.8 and 2.5 us, 57 x 35 x 30 2.0 and 3.0,
+// 131 x 67 x 45 3.1 and 5.1).
+// A set begins on a line of its own, so that clearing one touches no line of another that is being polled.
+constexpr int kCgSets = 4;
+__host__ __device__ constexpr unsigned post_stride(unsigned words) { return (words + 15u) & ~15u; }
+__device__ __forceinline__ u64 post_word(double v) {
+    const u64 u = (u64)__double_as_longlong(v);
+    return u ? u : 1ull << 63;
+}
+__device__ __forceinline__ double post_value(u64 u) { return __longlong_as_double((long long)u); }
+
 // Published row values of one vector: [2][n] (parity), FP32 as (value, tag) words.
 template <typename R>
 struct Pub;
@@ -294,6 +312,12 @@ __device__ __forceinline__ double rcp64(double d) {
     return fma(y, e, y);
 }
 
+// a / d from y = 1 / d to about an ulp: the quotient's remainder corrects it (Markstein 1990), rounded as a division's
+__device__ __forceinline__ double div64(double a, double d, double y) {
+    const double q = a * y;
+    return fma(fma(-d, q, a), y, q);
+}
+
 // Solver state of k_cg_local's iterations, held by every lane of wave 0 (all lanes compute the
 // same values from the same totals).
 struct CgRun {
@@ -365,7 +389,8 @@ struct BicgBlock {
     BlockKernel k;
     int together;
 };
-constexpr int kBicgSums = 9;  // sums of its largest reduction (posted: [4 reductions][2][kBicgSums][workgroup])
+constexpr int kBicgSums = 9;   // sums of its largest reduction
+constexpr int kBicgSets = 10;  // posted: one set per group of right-hand sides, then [3 reductions][2]; each [kBicgSums][post_stride(workgroups)]
 BicgBlock bicg_block(bool f32, int nz, int rpt, int nrhs);
 
 }  // namespace pict

@@ -2668,17 +2668,18 @@ long long block_wgs(long long n, long long C, int nz) { return ((nz <= 5 ? n : n
 
 // Bytes of k_cg_block's regions (the marks, one per tile of 8 rows, then from `off` the tagged partials and published
 // rows, zeroed before a launch) for nwg workgroups of C rows.
+size_t cg_post_words(long long nwg) { return (size_t)kCgSets * post_stride(2u * (unsigned)nwg); }
 size_t block_region(long long nwg, long long C, size_t &off) {
     const size_t pos = (size_t)nwg * C;
     off = (pos / 8 * sizeof(int) + 255) & ~size_t(255);
-    return 8 * ((size_t)nwg * 4 + 2 * pos);
+    return 8 * (cg_post_words(nwg) + 2 * pos);
 }
 // k_bicg_block's: the same, with `together` right-hand sides and larger reductions
-size_t bicg_tagged_words(long long nwg) { return (size_t)nwg * 8 * kBicgSums; }
+size_t bicg_post_words(long long nwg) { return (size_t)kBicgSets * kBicgSums * post_stride((unsigned)nwg); }
 size_t bicg_block_region(long long nwg, long long C, int together, size_t &off) {
     const size_t pos = (size_t)nwg * C;
     off = (pos / 8 * sizeof(int) + 255) & ~size_t(255);
-    return 8 * (bicg_tagged_words(nwg) + 2 * pos * together);
+    return 8 * (bicg_post_words(nwg) + 2 * pos * together);
 }
 
 // k_cg_block's shape for a system: instance and workgroups, or none (a longer row on average than its registers take,
@@ -3033,7 +3034,7 @@ pict_status enqueue_typed(const pict_csr_desc *A, const void *rhs, void *x, int 
         SolveArgs<R> ba = a;
         ba.p0 = (R *)ws;
         ba.tagged = (unsigned long long *)(ws + L.off_block);
-        ba.pub = ba.tagged + (kind == Kind::kBiCG ? bicg_tagged_words(pl.block_nwg) : (size_t)pl.block_nwg * 4);
+        ba.pub = ba.tagged + (kind == Kind::kBiCG ? bicg_post_words(pl.block_nwg) : cg_post_words(pl.block_nwg));
         ba.nwg = (unsigned)pl.block_nwg;
         ba.admit = admit_polls();
         ba.spin = spin_limit();
@@ -3374,7 +3375,7 @@ void fill_args(BatchSolve &b, int s, const pict_csr_desc &A, const void *rhs, vo
         ba.admit = kAdmitAlways;  // (a cooperative launch)
         ba.spin = kSpinLimit;
         ba.tagged = reinterpret_cast<unsigned long long *>(b.arena + off_blk[s]);
-        ba.pub = ba.tagged + (size_t)ba.nwg * 4;
+        ba.pub = ba.tagged + cg_post_words(ba.nwg);
         memcpy(b.bargs_host.data() + (size_t)s * sizeof ba, &ba, sizeof ba);
         a.gate = &a.ctl->zero_all;
     }
