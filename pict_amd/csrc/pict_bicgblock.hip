@@ -62,16 +62,17 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
     __shared__ R lv[BIG ? L : 1];      // BIG: v
     __shared__ int ltile[H / kTile];   // halo tile: position of its first row / kTile
     __shared__ double wsum[kSums][kBW], tot[kSums];
-    __shared__ int scan[kBW];
-    __shared__ unsigned key[2];
-    __shared__ BlockMap m;
+    __shared__ PlaceLds place;
+    __shared__ BlockMap smap;
     __shared__ int s_over, s_err, s_late, s_go;
     const unsigned bid = blockIdx.x;
     const int t = (int)threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     if (t == 0) s_over = s_err = s_late = 0;
-    block_map<T, C, NZ>(a.row, a.col, a.n, (int)a.nwg, m, key);
-    __syncthreads();
-    if (bid >= (unsigned)m.nwg) return;
+    int *mark = reinterpret_cast<int *>(a.p0);  // tiles that another workgroup reads (stamped with a.salt)
+    const int nh = block_place<T, C, H, RPT, NZ>(a.row, a.col, a.n, (int)a.nwg, bid, smap,
+                                                 reinterpret_cast<unsigned *>(&lr[0][0]), ltile, place, s_over, mark, a.salt);
+    if (nh < 0) return;
+    const BlockMap m = uniform_map(smap);
     const unsigned nwg = (unsigned)m.nwg;
     const unsigned first = bid * (unsigned)C;  // position of the first own row
     const size_t npos = (size_t)a.nwg * C;
@@ -86,31 +87,34 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
         if constexpr (kTagged) st_coh(elem(base, pos), ((u64)tag << 32) | (u64)__float_as_uint(v));
         else st_coh(elem(base, pos), v);
     };
-    int *mark = reinterpret_cast<int *>(a.p0);  // tiles that another workgroup reads (stamped with a.salt)
-    const int nh = block_halo<T, C, H, RPT, NO>(a.row, a.col, m, bid, reinterpret_cast<unsigned *>(&lr[0][0]), ltile,
-                                                scan, s_over, mark, a.salt);
 
     // ---- rows into registers ----
     R dv[RPT], val[RPT][NO];
     unsigned idx[RPT][NI];
+    // (in two parts: in one, the largest instance's loop is more than the compiler unrolls)
+    auto load_rows = [&](auto from) __attribute__((always_inline)) {
+        constexpr int Q0 = decltype(from)::value, Q1 = Q0 + 7 < RPT ? Q0 + 7 : RPT;
 #pragma unroll
-    for (int q = 0; q < RPT; ++q) {
-        const int li = t + q * T;
-        const int i = block_row<C>(m, bid, (unsigned)li);
-        const int ii = i < 0 ? 0 : i;
-        const int rs = *elem(a.row, ii);
-        const int len = i < 0 ? 0 : *elem(a.row, ii + 1) - rs;
-        block_load_row<C, H, NZ, false, BIG>(a, m, ii, li, first, rs, len,
-                                             reinterpret_cast<const unsigned *>(&lr[0][0]), dv[q], val[q], idx[q],
-                                             [](R, int) {});
-        // a row is finished before the next one is begun (else the unrolled rows' loads overlap and spill)
+        for (int q = Q0; q < Q1; ++q) {
+            const int li = t + q * T;
+            const int i = block_row<C, NZ>(m, bid, (unsigned)li);
+            const int ii = i < 0 ? 0 : i;
+            const int rs = *elem(a.row, ii);
+            const int len = i < 0 ? 0 : *elem(a.row, ii + 1) - rs;
+            block_load_row<C, H, NZ, false, BIG>(a, m, ii, li, first, rs, len,
+                                                 reinterpret_cast<const unsigned *>(&lr[0][0]), dv[q], val[q], idx[q],
+                                                 [](R, int) {});
+            // a row is finished before the next one is begun (else the unrolled rows' loads overlap and spill)
 #pragma unroll
-        for (int j = 0; j < NI; ++j) asm volatile("" : "+v"(idx[q][j]));
+            for (int j = 0; j < NI; ++j) asm volatile("" : "+v"(idx[q][j]));
 #pragma unroll
-        for (int j = 0; j < NO; ++j) asm volatile("" : "+v"(val[q][j]));
-        asm volatile("" : "+v"(dv[q])::"memory");
-        if constexpr (RPT >= 8) __builtin_amdgcn_sched_barrier(0);
-    }
+            for (int j = 0; j < NO; ++j) asm volatile("" : "+v"(val[q][j]));
+            asm volatile("" : "+v"(dv[q])::"memory");
+            if constexpr (RPT >= 8) __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    load_rows(std::integral_constant<int, 0>{});
+    if constexpr (RPT > 7) load_rows(std::integral_constant<int, 7>{});
     __syncthreads();  // the bitmap has been read
 
     // A z of own row q, z in `z` (own, then halo rows)
@@ -260,7 +264,9 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
         return any_halo ? (unsigned)(ltile[h0 / kTile + j * (kBF / kTile)] * kTile + h0 % kTile) : 0u;
     };
     static_assert(kBF % kTile == 0, "a thread's halo rows have the same place in their tiles");
-    constexpr bool kPosReg = RPT < 4;
+    // in registers where they fit (57 x 35 x 30, three right-hand sides: 130 us per solve, spilling, without 121; FP64 234
+    // and 193)
+    constexpr bool kPosReg = RPT < 4 && !(NR == 3 && RPT == 2);
     unsigned hpos[kPosReg ? HPT : 1];
     if constexpr (kPosReg) {
 #pragma unroll
@@ -316,7 +322,7 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
 #pragma unroll
             for (int q = 0; q < RPT; ++q) {
                 const int li = t + q * T;
-                const int i = block_row<C>(m, bid, ti + q * T);
+                const int i = block_row<C, NZ>(m, bid, ti + q * T);
                 const R x0 = i < 0 ? R(0) : *elem(xk, (unsigned)i);
                 lr[k][li] = x0;
                 if constexpr (BIG) xw[li] = x0;
@@ -327,7 +333,7 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
 #pragma unroll
                 for (int j = 0; j < HPT; ++j) {
                     const unsigned pos = halo_pos(j);
-                    const int i = block_row<C>(m, pos / C, pos % C);
+                    const int i = block_row<C, NZ>(m, pos / C, pos % C);
                     lr[k][C + h0 + j * kBF] = i < 0 ? R(0) : *elem(xk, (unsigned)i);
                     fence(j);
                 }
@@ -343,7 +349,7 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
 #pragma unroll
             for (int q = 0; q < RPT; ++q) {
                 const int li = t + q * T;
-                const int i = block_row<C>(m, bid, ti + q * T);
+                const int i = block_row<C, NZ>(m, bid, ti + q * T);
                 const R bv = i < 0 ? R(0) : *elem(bk, (unsigned)i);
                 const R rv = bv - product(lr[k], q);
                 tv[k][q] = rv;
@@ -363,7 +369,7 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
         if (group == 0) {
             for (int k = NR; k < a.nrhs; ++k)
                 for (int q = 0; q < RPT; ++q) {
-                    const int i = block_row<C>(m, bid, ti + q * T);
+                    const int i = block_row<C, NZ>(m, bid, ti + q * T);
                     if (i >= 0) acc0[NR] = fmax(acc0[NR], fabs((double)a.b[(size_t)k * a.n + i]));
                 }
             if (s_over) acc0[NR] = INFINITY;
@@ -385,7 +391,7 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
             if (a.zero_shortcut && bmax == 0.0) {
                 for (int k = 0; k < a.nrhs; ++k)
                     for (int q = 0; q < RPT; ++q) {
-                        const int i = block_row<C>(m, bid, ti + q * T);
+                        const int i = block_row<C, NZ>(m, bid, ti + q * T);
                         if (i >= 0) a.x[(size_t)k * a.n + i] = R(0);
                     }
                 if (bid == 0 && t < a.nrhs) cg1_init(a.st[t], 0.0, 1);
@@ -626,7 +632,7 @@ __global__ __launch_bounds__(512) void k_bicg_block(SolveArgs<R> a) {
 #pragma unroll
             for (int q = 0; q < RPT; ++q) {
                 const int li = t + q * T;
-                const int i = block_row<C>(m, bid, ti + q * T);
+                const int i = block_row<C, NZ>(m, bid, ti + q * T);
                 if (i >= 0) *elem(xk, (unsigned)i) = BIG ? xw[li] : x[k][BIG ? 0 : q];
                 fence(q);
             }

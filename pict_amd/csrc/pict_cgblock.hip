@@ -19,12 +19,13 @@
 // chunk would have most of its neighbours a plane away in other workgroups (192x96x96 on 256 workgroups:
 // 14,200 halo rows for 6,912 own rows), so the grid's line length and plane are read off the matrix (the
 // column offsets -d3, -d2, -1, 0, 1, d2, d3 of an interior row) and a workgroup owns a block of whole
-// lines (6 x 6 lines: 4,608 halo rows).  The mapping is a bijection of the rows whatever the matrix is:
-// a wrong guess costs halo rows, never correctness.
+// lines (6 x 6 lines: 4,608 halo rows).  Lines of which two are more than the halo holds (2-D: 448 to 890 cells,
+// 3-D: some 300) are cut into strips first (BlockMap).  The mapping is a bijection of the rows whatever the
+// matrix is: a wrong guess costs halo rows, never correctness.
 //
 // What bounds it: an iteration is one trip of the partial sums through memory (about 1.3 us between the XCDs for up to
 // 128 workgroups, 2 for 256), three workgroup barriers, and per row 0.25 us of LDS gathers and FP64 sums on a unit that
-// holds 14 of them per thread.  At 192 x 96 x 96 it takes 7.8 us where streaming the system takes 40 (184 MB at 4.6
+// holds 14 of them per thread.  At 192 x 96 x 96 it takes 7.3 us where streaming the system takes 40 (184 MB at 4.6
 // TB/s); figures for other sizes stand at plan_block (pict_solve.hip).
 //
 // A system of several workgroups that this kernel cannot hold (a longer row, too many halo rows, no block
@@ -143,9 +144,8 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
     __shared__ R lps[BIG ? 2 * C + 2 * H + WL * T : 1];
     __shared__ int ltile[ONE ? 1 : H / kTile + 1];  // halo tile: position of its first row / kTile
     __shared__ double wsum[2][2 * kBW];  // by generation parity: the waves' first sums, then their second
-    __shared__ int scan[kBW];
-    __shared__ unsigned key[2];
-    __shared__ BlockMap m;
+    __shared__ PlaceLds place;
+    __shared__ BlockMap smap;
     __shared__ int s_over, s_err, s_declined;
     struct Step {
         double alpha, beta;
@@ -155,14 +155,18 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
     // the wave number as a scalar: a wave takes its branch alone, without the other branch's waits
     const int t = (int)threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     if (t == 0) s_over = s_err = s_declined = 0;
+    int *mark = reinterpret_cast<int *>(a.p0);  // tiles that another workgroup reads (stamped with a.salt)
+    int nh = 0;                                 // halo rows (a multiple of kTile)
     if constexpr (ONE) {
-        if (t == 0) m = BlockMap{a.n, 1};
+        if (t == 0) smap = whole_map(a.n);
         __syncthreads();
     } else {
-        block_map<T, C, NZ>(a.row, a.col, a.n, (int)a.nwg, m, key);
-        __syncthreads();
-        if (bid >= (unsigned)m.nwg) return;
+        nh = block_place<T, C, H, RPT, NZ>(a.row, a.col, a.n, (int)a.nwg, bid, smap, reinterpret_cast<unsigned *>(lr),
+                                           ltile, place, s_over, mark, a.salt);
+        if (nh < 0) return;
     }
+    // (large instances leave the map in LDS: in scalar registers it spills those of the iterations, 8.5 instead of 7.4 us)
+    const std::conditional_t<BIG, const BlockMap &, const BlockMap> m = pick_map<BIG>(smap);
     const unsigned nwg = (unsigned)m.nwg;
     const unsigned first = bid * (unsigned)C;  // position of the first own row
     using PubT = decltype(Pub<R>::base);
@@ -172,63 +176,62 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
         if constexpr (kTagged) st_coh(elem(base, pos), ((u64)tag << 32) | (u64)__float_as_uint(v));
         else st_coh(elem(base, pos), v);
     };
-    int *mark = reinterpret_cast<int *>(a.p0);  // tiles that another workgroup reads (stamped with a.salt)
-    int nh = 0;                                 // halo rows (a multiple of kTile)
-
-    // ---- halo tiles ----
-    if constexpr (!ONE) {
-        nh = block_halo<T, C, H, RPT, NO>(a.row, a.col, m, bid, reinterpret_cast<unsigned *>(lr), ltile, scan, s_over, mark,
-                                          a.salt);
-    }
 
     // ---- rows into registers; r0 = b - A x0 ----
     R dv[RPT], val[RPT][NO], w[RPT], s[BIG ? 1 : RPT], x[BIG ? 1 : RPT], p[BIG ? 1 : RPT];
     unsigned idx[RPT][NI];
     unsigned longm = 0;  // bit q: row q is read from memory (ONE)
     double acc0 = 0.0, acc1 = 0.0;
+    // (in two parts: in one, the largest instance's loop is more than the compiler unrolls)
+    auto load_rows = [&](auto from) __attribute__((always_inline)) {
+        constexpr int Q0 = decltype(from)::value, Q1 = Q0 + 7 < RPT ? Q0 + 7 : RPT;
+        const BlockMap m = uniform_map(smap);
 #pragma unroll
-    for (int q = 0; q < RPT; ++q) {
-        const int li = t + q * T;
-        const int i = block_row<C>(m, bid, (unsigned)li);
-        const int ii = i < 0 ? 0 : i;
-        const int rs = *elem(a.row, ii);
-        int len = i < 0 ? 0 : *elem(a.row, ii + 1) - rs;
-        if constexpr (ONE) {
-            // a row of more entries than the registers hold is read from memory in every product
-            bool diag = false;
-            for (int e = 0; len >= NZ && e < NZ; ++e) diag |= a.col[rs + e] == ii;
-            if (len > NO + (diag ? 1 : 0)) {
-                longm |= 1u << q;
-                len = 0;
+        for (int q = Q0; q < Q1; ++q) {
+            const int li = t + q * T;
+            const int i = block_row<C, NZ>(m, bid, (unsigned)li);
+            const int ii = i < 0 ? 0 : i;
+            const int rs = *elem(a.row, ii);
+            int len = i < 0 ? 0 : *elem(a.row, ii + 1) - rs;
+            if constexpr (ONE) {
+                // a row of more entries than the registers hold is read from memory in every product
+                bool diag = false;
+                for (int e = 0; len >= NZ && e < NZ; ++e) diag |= a.col[rs + e] == ii;
+                if (len > NO + (diag ? 1 : 0)) {
+                    longm |= 1u << q;
+                    len = 0;
+                }
             }
-        }
-        const R x0 = i < 0 ? R(0) : *elem(a.x, ii), bv = i < 0 ? R(0) : *elem(a.b, ii);
-        R sum = 0;
-        block_load_row<C, H, NZ, ONE, BIG>(a, m, ii, li, first, rs, len, reinterpret_cast<const unsigned *>(lr), dv[q],
-                                           val[q], idx[q], [&](R v, int c) { sum += v * *elem(a.x, c); });
-        if constexpr (ONE)
-            if (longm >> q & 1u)
-                for (int e = rs; e < a.row[ii + 1]; ++e) sum += a.val[a.perm ? a.perm[e] : e] * a.x[a.col[e]];
-        const R rv = bv - sum;
-        w[q] = rv;  // until the bitmap in lr has been read
-        if constexpr (BIG) {
-            lps[li] = lps[C + li] = R(0);
-        } else {
-            x[q] = x0;
-            p[q] = s[q] = R(0);
-        }
-        if constexpr (!ONE) put_row(1, first + li, rv, 1u);  // every row: the marks are not known yet
-        acc0 += (double)rv * (double)rv;
-        acc1 = fmax(acc1, fabs((double)bv));
-        // a row is finished before the next one is begun (else the unrolled rows' loads and index arithmetic overlap
-        // and spill)
+            const R x0 = i < 0 ? R(0) : *elem(a.x, ii), bv = i < 0 ? R(0) : *elem(a.b, ii);
+            R sum = 0;
+            block_load_row<C, H, NZ, ONE, BIG>(a, m, ii, li, first, rs, len, reinterpret_cast<const unsigned *>(lr), dv[q],
+                                               val[q], idx[q], [&](R v, int c) { sum += v * *elem(a.x, c); });
+            if constexpr (ONE)
+                if (longm >> q & 1u)
+                    for (int e = rs; e < a.row[ii + 1]; ++e) sum += a.val[a.perm ? a.perm[e] : e] * a.x[a.col[e]];
+            const R rv = bv - sum;
+            w[q] = rv;  // until the bitmap in lr has been read
+            if constexpr (BIG) {
+                lps[li] = lps[C + li] = R(0);
+            } else {
+                x[q] = x0;
+                p[q] = s[q] = R(0);
+            }
+            if constexpr (!ONE) put_row(1, first + li, rv, 1u);  // every row: the marks are not known yet
+            acc0 += (double)rv * (double)rv;
+            acc1 = fmax(acc1, fabs((double)bv));
+            // a row is finished before the next one is begun (else the unrolled rows' loads and index arithmetic overlap
+            // and spill)
 #pragma unroll
-        for (int j = 0; j < NI; ++j) asm volatile("" : "+v"(idx[q][j]));
+            for (int j = 0; j < NI; ++j) asm volatile("" : "+v"(idx[q][j]));
 #pragma unroll
-        for (int j = 0; j < NO; ++j) asm volatile("" : "+v"(val[q][j]));
-        asm volatile("" : "+v"(dv[q]), "+v"(w[q])::"memory");
-        if constexpr (RPT >= 8) __builtin_amdgcn_sched_barrier(0);
-    }
+            for (int j = 0; j < NO; ++j) asm volatile("" : "+v"(val[q][j]));
+            asm volatile("" : "+v"(dv[q]), "+v"(w[q])::"memory");
+            if constexpr (RPT >= 8) __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    load_rows(std::integral_constant<int, 0>{});
+    if constexpr (RPT > 7) load_rows(std::integral_constant<int, 7>{});
     if constexpr (!ONE)
         if (s_over) acc1 = INFINITY;
     __syncthreads();  // the bitmap has been read
@@ -338,7 +341,7 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
         }
         if (a.zero_shortcut && t1 == 0.0) {
             for (int q = 0; q < RPT; ++q) {
-                const int i = block_row<C>(m, bid, (unsigned)(t + q * T));
+                const int i = block_row<C, NZ>(m, bid, (unsigned)(t + q * T));
                 if (i >= 0) a.x[i] = R(0);
             }
             if (bid == 0 && t == 0) cg1_init(a.st[0], t0, 1);
@@ -351,7 +354,7 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
     R *xw = reinterpret_cast<R *>(a.pub) + (size_t)a.nwg * C * (2 * sizeof(typename Pub<R>::Word) / sizeof(R)) + first;
     if constexpr (BIG) {
         for (int k = h0; k < C && wave > 0; k += kBF) {
-            const int i = block_row<C>(m, bid, (unsigned)k);
+            const int i = block_row<C, NZ>(m, bid, (unsigned)k);
             xw[k] = i < 0 ? R(0) : a.x[i];
         }
     }
@@ -573,14 +576,14 @@ __device__ __forceinline__ void cg_block(const SolveArgs<R> &a, unsigned bid) {
     }
     if constexpr (BIG) {
         for (int k = h0; k < C && wave > 0; k += kBF) {
-            const int i = block_row<C>(m, bid, (unsigned)k);
+            const int i = block_row<C, NZ>(m, bid, (unsigned)k);
             if (i >= 0) a.x[i] = xw[k];
         }
     }
 #pragma unroll
     for (int q = 0; q < (BIG ? 0 : RPT); ++q) {
         const int li = t + q * T;
-        const int i = block_row<C>(m, bid, (unsigned)li);
+        const int i = block_row<C, NZ>(m, bid, (unsigned)li);
         if (i < 0) continue;
         a.x[i] = x[q];
     }

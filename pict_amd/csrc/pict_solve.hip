@@ -2663,8 +2663,10 @@ struct Plan {
 };
 
 // Workgroups of k_cg_block for n rows, C rows each: as many as the rows fill; 3-D systems (7-entry rows) leave room
-// for blocks of whole grid lines.
-long long block_wgs(long long n, long long C, int nz) { return ((nz <= 5 ? n : n * 17 / 10) + C - 1) / C; }
+// for blocks of whole grid lines.  `strips`: 2-D systems for strips of long lines, which leave up to 4 % unused.
+long long block_wgs(long long n, long long C, int nz, bool strips = false) {
+    return ((nz > 5 ? n * 17 / 10 : strips ? n * 26 / 25 : n) + C - 1) / C;
+}
 
 // Bytes of k_cg_block's regions (the marks, one per tile of 8 rows, then from `off` the tagged partials and published
 // rows, zeroed before a launch) for nwg workgroups of C rows.
@@ -2689,11 +2691,13 @@ size_t bicg_block_region(long long nwg, long long C, int together, size_t &off) 
 //    barrier saves (80 x 80: 2.6 on one, 1.85 on 13).
 //  - 5-entry rows: one row per thread up to 64 workgroups, two up to 128 (256 x 256: 2.73 -> 1.8, the same on 64 and
 //    128 workgroups, 2.1 on 32 with four rows, 2.9 with eight); then four and eight as far as the compute units reach
-//    (640 x 500: 13.3 -> 3.0).  FP64 words carry no tag, so their exchange is not hidden and the gain small: two rows
-//    per thread from the start (97 x 61: 2.8 -> 2.4, 320 x 256: 3.8 -> 3.5, 200 x 150: 3.0 both).
+//    (640 x 500: 13.3 -> 3.0; lines cut into strips: 512 x 256 7.7 -> 1.86, 1024 x 128 17.9 -> 1.85, 1024 x 512 20.7 ->
+//    2.8, 1000 x 1000 24.5 -> 3.5).  FP64 words carry no tag, so their exchange is not hidden: two rows per thread from
+//    the start (97 x 61: 2.8 -> 2.3, 320 x 256: 3.8 -> 2.5).
 //  - 7-entry rows: the barrier grows past 128 workgroups (57 x 35 x 30: 2.6 on 199 with one row per thread, 1.95 on 99
 //    with two, 2.1 on 50 with four; before: 4.2), a row costs 0.25 us (131 x 67 x 45: 3.1 with four rows, 4.1 with
-//    eight; before: 17.2); 150 x 90 x 60: 25 -> 5.4, 192 x 96 x 96 with fourteen: 40 -> 7.8.
+//    eight; before: 17.2); 150 x 90 x 60: 25 -> 5.4, 192 x 96 x 96 with fourteen: 40 -> 7.3; lines cut into strips:
+//    400 x 10 x 9 8.6 -> 1.9, 512 x 64 x 48 36.7 -> 7.5.
 // PICT_CG_LOCAL_WGS (a workgroup budget of k_cg_local) selects plan_general's kernels.
 //
 // block_shape: instance and workgroups of a block kernel for n rows, the fewest rows per thread (kernel(rows): its
@@ -2718,6 +2722,7 @@ pict_status block_shape(long long n, int nz, int cus, F kernel, Plan &pl) {
         pict_status st = occupancy(k.kernel, occ, c, k.threads);
         if (st) return st;
         if (occ < 1) continue;
+        if (nz <= 5) nwg = std::min(cap, block_wgs(n, C, nz, true));  // (those without rows end at once)
         pl.block = k;
         pl.block_nwg = nwg;
         return PICT_OK;
@@ -2741,12 +2746,14 @@ pict_status plan_block(const pict_csr_desc *A, int cus, Plan &pl) {
 
 // k_bicg_block's shape for a system, by the same rule (its trips and rows cost the same, three and two times per
 // iteration).  Measured per solve from zero, all right-hand sides, before = the kernel of plan_general:
-//  - 5-entry rows, two right-hand sides together: 97 x 61 58 -> 37 us (2 iterations), 128 x 100 52 -> 41, 256 x 256 68
-//    -> 52 (65 with four rows per thread), 301 x 203 95 -> 53, 640 x 500 204 -> 109 (134 with eight); one after the
-//    other 1.2-1.4 times as much.  FP64 97 x 61 199 -> 57 (4 iterations), 320 x 256 186 -> 74, 640 x 500 279 -> 149.
+//  - 5-entry rows, two right-hand sides together: 97 x 61 58 -> 39 us (2 iterations), 128 x 100 52 -> 41, 256 x 256 68
+//    -> 48 (65 with four rows per thread), 301 x 203 95 -> 49, 640 x 500 204 -> 103 (134 with eight); one after the
+//    other 1.2-1.4 times as much.  FP64 97 x 61 199 -> 61 (4 iterations), 320 x 256 186 -> 74, 640 x 500 279 -> 126.
+//    Lines cut into strips: 512 x 256 110 -> 54, 1024 x 128 234 -> 72, 1000 x 1000 308 -> 152.
 //  - 7-entry rows, three together up to four rows per thread: 24 x 17 x 16 312 -> 91 (6 iterations; 148 one after the
-//    other), 57 x 35 x 30 325 -> 127 (204 with four rows), 131 x 67 x 45 617 -> 295 (361); one after the other 150 x 90
-//    x 60 1072 -> 529, 192 x 96 x 96 1864 -> 738.  FP64 57 x 35 x 30 563 -> 228, 90 x 60 x 40 852 -> 532.
+//    other), 57 x 35 x 30 325 -> 121 (204 with four rows), 131 x 67 x 45 617 -> 295 (361); one after the other 150 x 90
+//    x 60 1072 -> 529, 192 x 96 x 96 1864 -> 667, 512 x 64 x 48 (strips) 1405 -> 630.  FP64 57 x 35 x 30 563 -> 193,
+//    90 x 60 x 40 852 -> 532.
 // Systems of up to kBlockJobsOne rows stay with plan_general: a batch of them runs k_bicg_local_jobs, whose results a
 // single solve of the same system has to match to the bit, and 64 x 64 gains 8 us of 46 only.
 // PICT_BICG_LOCAL=0 and PICT_CG_LOCAL_WGS select plan_general's kernels.
@@ -3289,7 +3296,10 @@ bool plan_block_jobs(BatchSolve &b, bool f32, int most, long long cap) {
         const double t = rpt == 0 ? 0.6 + 0.7 * b.n[s] / kBlockJobsOne : rpt == 2 ? 1.8 : rpt == 4 ? 2.1 : 2.9;
         return t * std::sqrt((double)b.n[s]);
     };
-    auto wgs = [&](int s, int rpt) { return rpt == 0 ? 1LL : block_wgs(b.n[s], 512LL * rpt, b.nz); };
+    // (square grids have lines that are cut into strips from about 416 x 416 on)
+    auto wgs = [&](int s, int rpt) {
+        return rpt == 0 ? 1LL : block_wgs(b.n[s], 512LL * rpt, b.nz, b.n[s] >= 416 * 416);
+    };
     const long long sys_cap = std::min<long long>(cap, 256);
     double best = -1.0;
     std::vector<int> rpts(b.count), nwg(b.count);

@@ -53,3 +53,18 @@ def test_mixed_rows_match_single_steps(name, rows, dtype):
         r = np.linalg.norm(b.numpy() - m @ x.numpy())
         bound = tol * n + 16 * torch.finfo(dtype).eps * np.linalg.norm(abs(m) @ np.abs(x.numpy()))
         assert r <= bound, (n, r, bound)
+
+
+def test_long_lines():
+    """Systems whose grid lines are cut into strips, among shorter ones: held on chip in a batch too."""
+    sizes = [440, 512, 64, 500, 30]
+    doms, sims = _sims(sizes, torch.float32)
+    batch = SimulationBatch(sims)
+    for _ in range(2):
+        infos = batch.step()
+    assert (infos["reserved"][:, 2:] == 1).all() and (infos["converged"] == 1).all()
+    for n, d in zip(sizes, doms):
+        val, x, b = (t.detach().double().cpu().reshape(-1) for t in (d.P.value, d.pressureResult, d.pressureRHSdiv))
+        m = sp.csr_matrix((val.numpy(), d.P.index.cpu().numpy(), d.P.row.cpu().numpy()), shape=(n * n, n * n))
+        r = np.linalg.norm(b.numpy() - m @ x.numpy())
+        assert r <= 1e-6 * n + 16 * torch.finfo(torch.float32).eps * np.linalg.norm(abs(m) @ np.abs(x.numpy())), n

@@ -1,6 +1,7 @@
 """k_cg_block, the CG with a system's whole state on chip (the default for one right-hand side and a norm-2 criterion):
 sizes on both sides of every line where another instance or workgroup count is chosen, one workgroup and several, grids
 whose lines do not fill tiles or workgroups, 3-D blocks of lines that end inside the grid, transposed solves, and
+lines longer than the halo (cut into strips),
 systems it leaves to the general kernels (long rows, too many foreign columns), against a direct FP64 solve and the
 general kernels (PICT_CG_LOCAL_WGS selects them).
 
@@ -43,9 +44,10 @@ def check(m, dtype, name_part, monkeypatch, seed=3, on_chip=True):
     tol = 1e-12 if dtype == torch.float64 else 1e-6
     x, info = solve(A, b, tol)
     assert info.converged and info.isFiniteResidual
-    assert info.onChip == on_chip  # which kernel solved it, not only which one was planned
+    assert on_chip is None or info.onChip == on_chip  # which kernel solved it, not only which one was planned
     x2, info2 = solve(A, b, tol)
-    assert info2.usedIterations == info.usedIterations and torch.equal(x, x2)
+    # (the general FP64 kernel may put other rows in memory from run to run when lines are as long as its workgroups)
+    assert info2.usedIterations == info.usedIterations and (torch.equal(x, x2) or (on_chip is None and not info.onChip))
     monkeypatch.setenv("PICT_CG_LOCAL_WGS", "64")
     xr, ir = solve(A, b, tol)
     assert not ir.onChip
@@ -81,13 +83,12 @@ def test_one_workgroup_1024_threads(shape, monkeypatch):
 def test_several_workgroups_2d(shape, rpt, build, monkeypatch):
     if build is periodic_laplacian and min(shape) < 3:
         shape = (1366, 3)
-    # (two whole lines are more than the 896 halo rows from 449 cells on)
-    check(build(shape, 0.05), torch.float32, "512, %d, 5, several" % rpt, monkeypatch, on_chip=2 * shape[0] <= 896 or shape[1] == 1)
+    check(build(shape, 0.05), torch.float32, "512, %d, 5, several" % rpt, monkeypatch)
 
 
 @pytest.mark.parametrize("shape", [(683, 4), (97, 61), (181, 182)])
 def test_several_workgroups_2d_fp64(shape, monkeypatch):
-    check(walls(shape, 0.05), torch.float64, "several", monkeypatch, on_chip=2 * shape[0] <= 896)
+    check(walls(shape, 0.05), torch.float64, "several", monkeypatch)
 
 
 # 3-D: blocks of lines that do not divide the grid, planes larger and smaller than a workgroup
@@ -102,11 +103,43 @@ def test_several_workgroups_3d_fp64(shape, monkeypatch):
     check(periodic_laplacian(shape, 0.05), torch.float64, "several", monkeypatch)
 
 
+# lines that leave no room for two of them in the halo (896, 1344 and 1792 rows) are cut into strips
+@pytest.mark.parametrize("shape,rpt", [((400, 70), 1), ((449, 70), 1), ((512, 64), 1), ((1500, 21), 1), ((512, 128), 2),
+                                       ((1000, 100), 2), ((640, 300), 4), ((700, 300), 4), ((700, 400), 4),
+                                       ((890, 700), 8), ((897, 700), 8), ((1000, 1000), 8), ((1024, 1024), 8)])
+@pytest.mark.parametrize("build", [walls, periodic_laplacian])
+def test_strips_2d(shape, rpt, build, monkeypatch):
+    if shape[0] * shape[1] > 500000 and build is periodic_laplacian and shape[0] != 1000:
+        pytest.skip("large: once")
+    check(build(shape, 0.05), torch.float32, "512, %d, 5, several" % rpt, monkeypatch)
+
+
+@pytest.mark.parametrize("shape", [(1000, 50), (1000, 300)])
+def test_strips_2d_fp64(shape, monkeypatch):
+    check(periodic_laplacian(shape, 0.05), torch.float64, "several", monkeypatch)
+
+
+@pytest.mark.parametrize("shape,rpt", [((400, 10, 9), 1), ((1000, 9, 8), 2), ((700, 13, 15), 4), ((800, 23, 30), 8),
+                                       ((512, 48, 40), 14)])
+def test_strips_3d(shape, rpt, monkeypatch):
+    check(walls(shape, 0.05), torch.float32, "512, %d, 7, several" % rpt, monkeypatch)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_blocks_of_different_lines(dtype, monkeypatch):
+    """A domain of blocks with lines of different lengths: whichever the mapping follows, the answer is right."""
+    for shapes in (((600, 40), (90, 100)), ((90, 100), (600, 40)), ((30, 20, 20), (600, 5, 4)), ((600, 5, 4), (30, 20, 20))):
+        m = sp.block_diag([walls(s, 0.05) for s in shapes]).tocsr()
+        m.sort_indices()
+        check(m, dtype, "several", monkeypatch, on_chip=None)
+
+
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 def test_left_to_the_general_kernel(dtype, monkeypatch):
-    """Lines too long for the halo, columns all over the system, and rows longer than the registers: the general
-    kernel solves them; on one workgroup long rows are read from memory."""
-    check(walls((3000, 4), 0.05), dtype, "several", monkeypatch, on_chip=False)
+    """Two long lines (no interior row shows their length), columns all over the system, and rows longer than the
+    registers: the general kernel solves them; on one workgroup long rows are read from memory."""
+    check(walls((3000, 2), 0.05), dtype, "several", monkeypatch, on_chip=dtype == torch.float32)  # (512 and 1024 rows)
+    check(walls((3000, 4), 0.05), dtype, "several", monkeypatch)
     check(irregular(20000, 3), dtype, "", monkeypatch, on_chip=False)
     n = 12000
     m = walls((120, 100), 0.05).tolil()
