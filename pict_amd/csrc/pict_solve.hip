@@ -30,6 +30,7 @@
 #include <vector>
 
 #include "pict_krylov.hpp"
+#include "pict_schedule.hpp"
 
 namespace pict {
 
@@ -3146,7 +3147,6 @@ struct BatchSolve {
     char *arena = nullptr;
     std::vector<char> args_host;
     std::vector<unsigned> job_off, jobs;
-    double makespan = 0.0;
     // k_cg_block_jobs in front (null: none) with its own workgroups, lists and argument table; the kernel above is
     // queued behind it for the systems it cannot hold
     const void *block = nullptr;
@@ -3216,44 +3216,11 @@ __global__ __launch_bounds__(256) void k_batch_err(const SolveArgs<R> *args, int
     if (threadIdx.x == 0) *out = any;
 }
 
-// List scheduling of the systems' jobs onto `grid` workgroups (cost: estimated time of each solve); returns the
-// makespan.
-double schedule(int count, const std::vector<int> &nwg, unsigned grid, const std::vector<double> &cost,
-                std::vector<unsigned> &job_off, std::vector<unsigned> &jobs) {
-    std::vector<int> order(count);
-    for (int s = 0; s < count; ++s) order[s] = s;
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cost[x] > cost[y]; });
-    std::vector<double> avail(grid, 0.0);
-    std::vector<std::vector<unsigned>> lists(grid);
-    std::vector<unsigned> idx(grid);
-    double makespan = 0.0;
-    for (int s : order) {
-        const unsigned k = (unsigned)nwg[s];
-        for (unsigned g = 0; g < grid; ++g) idx[g] = g;
-        auto earlier = [&](unsigned x, unsigned y) { return avail[x] < avail[y] || (avail[x] == avail[y] && x < y); };
-        std::nth_element(idx.begin(), idx.begin() + (k - 1), idx.end(), earlier);
-        std::sort(idx.begin(), idx.begin() + k);
-        double start = 0.0;
-        for (unsigned j = 0; j < k; ++j) start = std::max(start, avail[idx[j]]);
-        const double fin = start + cost[s];
-        for (unsigned j = 0; j < k; ++j) {
-            lists[idx[j]].push_back(((unsigned)s << 16) | j);
-            avail[idx[j]] = fin;
-        }
-        makespan = std::max(makespan, fin);
-    }
-    job_off.assign(grid + 1, 0);
-    jobs.clear();
-    for (unsigned g = 0; g < grid; ++g) {
-        job_off[g] = (unsigned)jobs.size();
-        jobs.insert(jobs.end(), lists[g].begin(), lists[g].end());
-    }
-    job_off[grid] = (unsigned)jobs.size();
-    return makespan;
-}
+// cost: of each solve in iterations, by size or measured
 void schedule(BatchSolve &b, const std::vector<double> &cost) {
-    b.makespan = schedule(b.count, b.nwg, b.grid, cost, b.job_off, b.jobs);
-    if (b.block) b.makespan = schedule(b.count, b.block_nwg, b.block_grid, cost, b.bjob_off, b.bjobs);
+    schedule(b.count, b.nwg, b.grid, cost, b.job_off, b.jobs);
+    if (b.block)
+        schedule(b.count, b.block_nwg, b.block_grid, block_job_costs(b.n, b.block_rpt, cost), b.bjob_off, b.bjobs);
 }
 // the argument and job tables to the device, in stream order
 pict_status upload_jobs(const BatchSolve &b, hipStream_t stream) {
@@ -3291,11 +3258,7 @@ std::vector<double> default_cost(const BatchSolve &b) {
 // for the system that takes longest.  64 lid cavities of 32 x 32 to 248 x 248 (720 iterations): 2.3 ms with four rows for
 // all, in two rounds, 2.5 ms with eight in one, 1.7 ms with this plan.
 bool plan_block_jobs(BatchSolve &b, bool f32, int most, long long cap) {
-    // us per iteration (256 x 256 on 32 workgroups and more), one workgroup: by rows; iterations like the square root
-    auto cost = [&](int s, int rpt) {
-        const double t = rpt == 0 ? 0.6 + 0.7 * b.n[s] / kBlockJobsOne : rpt == 2 ? 1.8 : rpt == 4 ? 2.1 : 2.9;
-        return t * std::sqrt((double)b.n[s]);
-    };
+    auto cost = [&](int s, int rpt) { return block_job_us(b.n[s], rpt) * std::sqrt((double)b.n[s]); };
     // (square grids have lines that are cut into strips from about 416 x 416 on)
     auto wgs = [&](int s, int rpt) {
         return rpt == 0 ? 1LL : block_wgs(b.n[s], 512LL * rpt, b.nz, b.n[s] >= 416 * 416);
@@ -3638,7 +3601,6 @@ void batch_solve_describe(const BatchSolve *b, BatchSolveInfo *out) {
     out->rows_per_wg = b->rows_per_wg;
     out->local = b->local || b->bicg_local ? 1 : 0;
     out->jobs = (int)(b->block ? b->bjobs.size() : b->jobs.size());
-    out->makespan = b->makespan;
     const bool f32 = b->dtype == PICT_DTYPE_F32;
     if (b->block)
         snprintf(out->kernel, sizeof out->kernel, "pict::k_cg_block_jobs<%s, %d>", f32 ? "float" : "double", b->nz);

@@ -43,7 +43,6 @@ struct BatchSolveConfig {
 
 struct BatchSolveInfo {
     int grid, rows_per_thread, rows_per_wg, local, jobs;
-    double makespan;  // of the schedule, in units of the cost estimates
     char kernel[64];
 };
 
