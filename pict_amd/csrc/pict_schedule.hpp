@@ -9,7 +9,7 @@ namespace pict {
 
 // List scheduling of the systems' jobs onto `grid` workgroups (cost: estimated time of each solve); returns the
 // makespan.
-inline double schedule(int count, const std::vector<int> &nwg, unsigned grid, const std::vector<double> &cost,
+inline double list_schedule(int count, const std::vector<int> &nwg, unsigned grid, const std::vector<double> &cost,
                 std::vector<unsigned> &job_off, std::vector<unsigned> &jobs) {
     std::vector<int> order(count);
     for (int s = 0; s < count; ++s) order[s] = s;

@@ -3218,9 +3218,9 @@ __global__ __launch_bounds__(256) void k_batch_err(const SolveArgs<R> *args, int
 
 // cost: of each solve in iterations, by size or measured
 void schedule(BatchSolve &b, const std::vector<double> &cost) {
-    schedule(b.count, b.nwg, b.grid, cost, b.job_off, b.jobs);
+    list_schedule(b.count, b.nwg, b.grid, cost, b.job_off, b.jobs);
     if (b.block)
-        schedule(b.count, b.block_nwg, b.block_grid, block_job_costs(b.n, b.block_rpt, cost), b.bjob_off, b.bjobs);
+        list_schedule(b.count, b.block_nwg, b.block_grid, block_job_costs(b.n, b.block_rpt, cost), b.bjob_off, b.bjobs);
 }
 // the argument and job tables to the device, in stream order
 pict_status upload_jobs(const BatchSolve &b, hipStream_t stream) {
@@ -3277,7 +3277,7 @@ bool plan_block_jobs(BatchSolve &b, bool f32, int most, long long cap) {
             costs[s] = cost(s, rpts[s]);
             sum += w;
         }
-        const double m = schedule(b.count, nwg, (unsigned)std::min(sum, cap), costs, off, jobs);
+        const double m = list_schedule(b.count, nwg, (unsigned)std::min(sum, cap), costs, off, jobs);
         if (best >= 0.0 && m >= best) return false;
         best = m;
         b.block_nwg = nwg;

@@ -17,7 +17,7 @@ int main() {
     const std::vector<double> it{800, 300, 500, 280, 310};
     std::vector<unsigned> off, jobs;
     const auto us = block_job_costs(n, rpt, it);
-    const double makespan = schedule(5, nwg, 20, us, off, jobs);
+    const double makespan = list_schedule(5, nwg, 20, us, off, jobs);
     printf("%.1f\n", makespan);
     for (double u : us) printf("%.1f ", u);
     printf("\n");
