@@ -489,7 +489,8 @@ typedef struct pict_batch pict_batch;
 typedef struct pict_batch_config {
     int32_t tiles_per_workgroup;        /* 256-cell tiles per workgroup of the stage kernels: 1, 2 or 4 */
     int32_t pressure_rows_per_thread;   /* CG: matrix rows each thread keeps in registers: 1, 2, 4, 8
-                                           (the on-chip kernel: at most so many, chosen per system)  */
+                                           (the on-chip kernel: at most so many, chosen per system;
+                                           for 1 two)                                                */
     int32_t advection_rows_per_workgroup; /* BiCGStab: rows per workgroup (>= 64)                     */
     int32_t adaptive_schedule;          /* 1: after the first step, schedule the solves by the
                                            iteration counts it took; 0: by system size only         */

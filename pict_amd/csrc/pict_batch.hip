@@ -396,17 +396,21 @@ pict_status collect(pict_batch *b, const pict_step_opts *o, pict_solve_info *inf
     // after the first step: schedule the solves by the iterations they took
     if (p.cfg.adaptive_schedule && !p.rescheduled) {
         std::vector<double> ca(b->count), cp(b->count);
+        bool on_chip = true;
         for (int d = 0; d < b->count; ++d) {
             int ia = 1, ip = 1;
             for (int c = 0; c < D; ++c) ia = std::max(ia, infos[(size_t)d * per + c].used_iterations + 1);
-            for (int k = 0; k < K; ++k) ip = std::max(ip, infos[(size_t)d * per + D + k].used_iterations + 1);
+            for (int k = 0; k < K; ++k) {
+                ip = std::max(ip, infos[(size_t)d * per + D + k].used_iterations + 1);
+                on_chip = on_chip && infos[(size_t)d * per + D + k].reserved == 1;
+            }
             const int na = b->atlases[d]->desc.num_cells;
             ca[d] = (double)ia * (2048.0 + (double)na / std::max(1, (na + 1023) / 1024));
             cp[d] = (double)ip;
         }
-        pict_status st = batch_solve_reschedule(p.adv, ca.data(), s);
+        pict_status st = batch_solve_reschedule(p.adv, ca.data(), false, s);
         if (st) return st;
-        if (K > 0 && (st = batch_solve_reschedule(p.prs, cp.data(), s))) return st;
+        if (K > 0 && (st = batch_solve_reschedule(p.prs, cp.data(), on_chip, s))) return st;
         p.rescheduled = true;
     }
     return PICT_OK;

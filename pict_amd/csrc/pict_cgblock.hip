@@ -636,7 +636,7 @@ __global__ __launch_bounds__(512) void k_cg_block_jobs(const SolveArgs<R> *__res
     }
 }
 
-// Instances.  One workgroup: up to 1024 threads x 8 rows; several: 512 threads.
+// Instances.  One workgroup: up to 512 threads x 4 rows, FP32 1024 x 4; several: 512 threads.
 template <typename R, int NZ>
 static BlockKernel one_kernel(long long n) {
     constexpr bool f32 = sizeof(R) == 4;

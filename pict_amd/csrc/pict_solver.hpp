@@ -56,8 +56,8 @@ void batch_solve_destroy(BatchSolve *b);
 // new matrix or vector addresses (same sizes); waits for queued work when the table changes
 pict_status batch_solve_update(BatchSolve *b, const pict_csr_desc *A, const void *const *rhs, void *const *x,
                                hipStream_t stream);
-// new schedule from measured costs (waits for queued work)
-pict_status batch_solve_reschedule(BatchSolve *b, const double *cost, hipStream_t stream);
+// new schedule from measured costs (waits for queued work); on_chip: the block kernel has solved every system
+pict_status batch_solve_reschedule(BatchSolve *b, const double *cost, bool on_chip, hipStream_t stream);
 // Queues the solves (no allocation, no host wait: capturable).  states_out (may be null): count*nrhs
 // final states (solve_state_bytes() each); err_out (may be null): nonzero when a barrier timed out.
 pict_status batch_solve_enqueue(const BatchSolve *b, void *states_out, int *err_out, hipEvent_t ev0, hipEvent_t ev1,

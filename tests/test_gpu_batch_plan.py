@@ -10,6 +10,7 @@ import pytest
 import scipy.sparse as sp
 import torch
 
+from pict_amd import PISOtorch as P
 from pict_amd import PISOtorch_simulation as S
 from pict_amd import configs
 from pict_amd.batch import SimulationBatch
@@ -68,3 +69,39 @@ def test_long_lines():
         m = sp.csr_matrix((val.numpy(), d.P.index.cpu().numpy(), d.P.row.cpu().numpy()), shape=(n * n, n * n))
         r = np.linalg.norm(b.numpy() - m @ x.numpy())
         assert r <= 1e-6 * n + 16 * torch.finfo(torch.float32).eps * np.linalg.norm(abs(m) @ np.abs(x.numpy())), n
+
+
+def _two_boxes(shapes, dtype, name):
+    """Closed boxes side by side, not connected: one domain whose grid lines have different lengths."""
+    dom = P.Domain(2, torch.tensor([0.01], dtype=dtype), name, dtype, "cuda", passiveScalarChannels=0)
+    g = torch.Generator().manual_seed(5)
+    for k, (nx, ny) in enumerate(shapes):
+        x = torch.linspace(0, 1, nx + 1, dtype=dtype) + 2 * k
+        y = torch.linspace(0, 1, ny + 1, dtype=dtype)
+        yy, xx = torch.meshgrid(y, x, indexing="ij")
+        b = dom.CreateBlock(vertexCoordinates=torch.stack([xx, yy])[None].cuda().contiguous(), name="b%d" % k)
+        b.CloseAllBoundaries()
+        b.setVelocity((0.05 * torch.randn(1, 2, ny, nx, generator=g, dtype=torch.float64)).to(dtype).cuda())
+    dom.PrepareSolve()
+    return dom
+
+
+def test_a_system_left_to_the_general_kernel():
+    """One system of a batch that the on-chip kernel does not hold (its first lines are 90 cells, others 1000): the general
+    kernel solves it in every step, captured ones included, and the others stay on chip."""
+    shapes = [[(64, 64)], [(90, 300), (1000, 30)], [(100, 90)]]
+    doms = [_two_boxes(s, torch.float32, "d%d" % i) for i, s in enumerate(shapes)]
+    sims = [S.Simulation(d, time_step=1e-3, corrector_steps=2, non_orthogonal=False, advection_tol=1e-6,
+                         pressure_tol=1e-6, advect_passive_scalar=False) for d in doms]
+    batch = SimulationBatch(sims)
+    for _ in range(5):
+        infos = batch.step()
+        assert (infos["converged"] == 1).all()
+        assert infos["reserved"][:, 2:].tolist() == [[1, 1], [0, 0], [1, 1]]
+        for d in doms:
+            val, x, b = (t.detach().double().cpu().reshape(-1) for t in (d.P.value, d.pressureResult, d.pressureRHSdiv))
+            n = b.numel()
+            m = sp.csr_matrix((val.numpy(), d.P.index.cpu().numpy(), d.P.row.cpu().numpy()), shape=(n, n))
+            r = np.linalg.norm(b.numpy() - m @ x.numpy())
+            bound = 1e-6 * np.sqrt(n) + 16 * torch.finfo(torch.float32).eps * np.linalg.norm(abs(m) @ np.abs(x.numpy()))
+            assert r <= bound, (n, r, bound)
