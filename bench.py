@@ -55,6 +55,33 @@ def solver_bytes(kind, n, nnz, nrhs, s, iters):
     return sum(max(it, 0) * per_it + spmv + n * s for it in iters)
 
 
+def solver_bytes_once(n, nnz, nrhs, s):
+    """What a solve that keeps its system on chip has to move: the matrix and right-hand sides read once, the solutions
+    read and written once."""
+    return nnz * (s + 4) + (n + 1) * 4 + 3 * nrhs * n * s
+
+
+def on_chip(kernel):
+    """A solver kernel that holds matrix and vectors on chip while it iterates (k_cg_block, k_bicg_block, their batched
+    form)."""
+    return "_block" in kernel
+
+
+def solver_roofline(kernel, bytes_iterated, bytes_once, avg_ms, iterations, traffic, traffic_source, **more):
+    """The roofline entry of a solver kernel.  One that streams its system moves bytes_iterated per launch and is held
+    against the HBM rate.  One that keeps it on chip moves bytes_once, and its time is the chain of its reductions:
+    iterations of a launch, one after the other (of a batch: of its longest system)."""
+    b = bytes_once if on_chip(kernel) else bytes_iterated
+    achieved = b / (avg_ms * 1e-3) / 1e9
+    out = {"bound": "latency" if on_chip(kernel) else "hbm", "kernel": kernel, "achieved": achieved,
+           "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
+           "traffic_source": traffic_source, "bytes_per_launch": b, "avg_launch_ms": avg_ms}
+    if on_chip(kernel):
+        out["us_per_iteration"] = avg_ms * 1e3 / max(iterations, 1.0)
+    out.update(more)
+    return out
+
+
 def make_workload(args, torch, dtype=None):
     from pict_amd import PISOtorch_simulation as S
     from pict_amd import configs
@@ -242,8 +269,11 @@ def main():
     # per-kernel roofline from the solver log
     agg = {}
     for kind, n, nnz, nrhs, s, infos, kms, transposed, name in log:
-        a = agg.setdefault(name, {"ms": 0.0, "bytes": 0, "launches": 0, "iters": 0, "adjoint_launches": 0})
+        a = agg.setdefault(name, {"ms": 0.0, "bytes": 0, "once": 0, "launches": 0, "iters": 0, "chain": 0,
+                                  "adjoint_launches": 0})
         its = [i.usedIterations + 1 for i in infos]
+        a["once"] += solver_bytes_once(n, nnz, nrhs, s)
+        a["chain"] += max(its)
         a["ms"] += kms
         a["bytes"] += solver_bytes(kind, n, nnz, nrhs, s, its)
         a["launches"] += 1
@@ -252,8 +282,6 @@ def main():
     dom_kernel = max(agg, key=lambda k: agg[k]["ms"])
     d = agg[dom_kernel]
     avg_ms = d["ms"] / d["launches"]
-    bytes_per_launch = d["bytes"] / d["launches"]
-    achieved = bytes_per_launch / (avg_ms * 1e-3) / 1e9
     ms_per_step = ms_total / args.steps
     value = N * args.steps / (ms_total * 1e-3)
 
@@ -324,9 +352,8 @@ def main():
                    "solver_iterations_per_step": {k: v["iters"] / args.steps for k, v in agg.items()},
                    "solver_ms_per_step": {k: v["ms"] / args.steps for k, v in agg.items()},
                    "wall_s": wall, **extra},
-        "roofline": {"bound": "hbm", "kernel": dom_kernel, "achieved": achieved, "peak": HBM_PEAK_GBS,
-                     "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                     "traffic_source": traffic_source, "bytes_per_launch": bytes_per_launch, "avg_launch_ms": avg_ms},
+        "roofline": solver_roofline(dom_kernel, d["bytes"] / d["launches"], d["once"] / d["launches"], avg_ms,
+                                    d["chain"] / d["launches"], traffic, traffic_source),
         "cpu_baseline": cpu,
     }
     if batched is not None:
@@ -402,8 +429,10 @@ def bench_c2(args, torch):
     P.enable_solve_log(False)
     agg = {}
     for kind, n, nnz, nrhs, s_, inf, kms, transposed, name in log:
-        a = agg.setdefault(name, {"ms": 0.0, "bytes": 0, "launches": 0, "iters": 0})
+        a = agg.setdefault(name, {"ms": 0.0, "bytes": 0, "once": 0, "launches": 0, "iters": 0, "chain": 0})
         its = [i.usedIterations + 1 for i in inf]
+        a["once"] += solver_bytes_once(n, nnz, nrhs, s_)
+        a["chain"] += max(its)
         a["ms"] += kms
         a["bytes"] += solver_bytes(kind, n, nnz, nrhs, s_, its)
         a["launches"] += 1
@@ -412,7 +441,6 @@ def bench_c2(args, torch):
     d = agg[dk]
     avg_ms = d["ms"] / d["launches"]
     bpl = d["bytes"] / d["launches"]
-    achieved = bpl / (avg_ms * 1e-3) / 1e9
     cpu = None if args.no_cpu_baseline else cpu_baseline_c2(args)
     return {
         "metric": "cells*PISO-steps/s (forward)",
@@ -437,9 +465,7 @@ def bench_c2(args, torch):
                                            "pressure_inner": sum(p_its) / args.steps},
                    "solver_ms_per_step": {k: v["ms"] / 2 for k, v in agg.items()},
                    "solver_launches_per_step": {k: v["launches"] / 2 for k, v in agg.items()}},
-        "roofline": {"bound": "hbm", "kernel": dk, "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBS, "traffic": None, "bytes_per_launch": bpl,
-                     "avg_launch_ms": avg_ms},
+        "roofline": solver_roofline(dk, bpl, d["once"] / d["launches"], avg_ms, d["chain"] / d["launches"], None, None),
         "cpu_baseline": cpu,
     }
 
@@ -766,7 +792,7 @@ def bench_c4(args, torch):
         return sum(solver_bytes("CG", d.getTotalSize(), d.C.getSize(), 1, 4, [int(used[i][2 + k]) + 1])
                    for i, d in enumerate(doms_b))
     batch.set_timing(True)
-    l_ms, l_bytes, kms_all = [], [], []
+    l_ms, l_bytes, l_chain, kms_all = [], [], [], []
     for _ in range(max(1, args.roofline_steps)):
         arr = batch.step()
         kms = batch.last_solve_ms()
@@ -774,13 +800,16 @@ def bench_c4(args, torch):
         for k in range(K):
             l_ms.append(kms[1 + k])
             l_bytes.append(launch_bytes(arr["used_iterations"], k))
+            l_chain.append(int(arr["used_iterations"][:, 2 + k].max()) + 1)
     batch.set_timing(False)
     kms = [float(np.mean([x[j] for x in kms_all])) for j in range(len(kms_all[0]))]
     avg_ms = float(np.mean(l_ms))
     bytes_per_launch = float(np.mean(l_bytes))
-    achieved = bytes_per_launch / (avg_ms * 1e-3) / 1e9
+    bytes_once = float(sum(solver_bytes_once(d.getTotalSize(), d.C.getSize(), 1, 4) for d in doms_b))
+    chain = float(np.mean(l_chain))
     # the same model over the timed (graph-replayed) steps, for a kernel trace of them
-    timed_bytes_per_launch = float(np.mean([launch_bytes(u, k) for u in iters for k in range(K)]))
+    timed_bytes_per_launch = bytes_once if on_chip(info["pressure_kernel"]) else \
+        float(np.mean([launch_bytes(u, k) for u in iters for k in range(K)]))
     traffic, traffic_source = None, None
     if args.pmc_fetch and args.pmc_write:
         traffic, traffic_source = pmc_traffic(args.pmc_fetch, args.pmc_write, info["pressure_kernel"]), "counter files"
@@ -827,10 +856,8 @@ def bench_c4(args, torch):
                                            "pressure_max": int(its[:, :, 2:].max()),
                                            "pressure_sum": float(its[:, :, 2:].sum() / args.steps)},
                    "solver_ms_per_step": {"advection": kms[0], "pressure": sum(kms[1:])}},
-        "roofline": {"bound": "hbm", "kernel": info["pressure_kernel"], "achieved": achieved, "peak": HBM_PEAK_GBS,
-                     "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                     "traffic_source": traffic_source, "bytes_per_launch": bytes_per_launch, "avg_launch_ms": avg_ms,
-                     "launches": len(l_ms), "timed_bytes_per_launch": timed_bytes_per_launch},
+        "roofline": solver_roofline(info["pressure_kernel"], bytes_per_launch, bytes_once, avg_ms, chain, traffic,
+                                    traffic_source, launches=len(l_ms), timed_bytes_per_launch=timed_bytes_per_launch),
         "cpu_baseline": cpu,
     }
 
@@ -862,7 +889,8 @@ def pmc_traffic(fetch_csv, write_csv, kernel):
                     continue
                 name = r["Kernel_Name"].replace("void ", "").split("(")[0]
                 v = float(r["Counter_Value"])
-                if name == kernel:
+                if name == kernel or (on_chip(kernel) and "_jobs" not in kernel and
+                                      name.startswith(kernel.rsplit(",", 1)[0])):
                     vals.append(v)
                 elif "copyBuffer" in name:
                     copy = max(copy, v)
